@@ -222,6 +222,38 @@ int tq_attention_fwd_kv(const uint16_t* q_rot, const float* q_proj,
                         int64_t soh, int64_t sos, void* workspace,
                         int64_t workspace_bytes, void* stream);
 
+/* Fused attention for many query rows (prefill, prompt chunks) from raw queries
+ * q[B, Hq, Sq, d] (element strides; unit stride on d): query rotation, scores, softmax, P.V
+ * and output rotation, the whole tail of tq_query_prep + tq_attention_fwd_kv in one call.  The
+ * estimator is linear in the rotated query, so each key is expanded once to
+ *   k^ = vn Ck[codes] + coeff rn S_eff^T (2*sign - 1),   score = <q_rot, k^>,
+ * (f32 grade: f16 hi + lo parts) instead of projecting every query; key_s_eff_f16 is the same
+ * f16[d, d] table tq_query_prep takes.  Other operands as in tq_attention_fwd_kv; the mask is
+ * read in its own type (mask_dtype); out is contiguous [B, Sq, Hq, d].  `workspace` (16-byte aligned) holds the rotated queries and the
+ * expanded keys and values: tq_prefill_workspace_size bytes run every (batch, kv head) at
+ * once up to 1 GiB of expanded planes and the rest in further rounds over the same memory.
+ * Replaces the family forward tail families/qwen2.py:105-117, as tq_attention_fwd. */
+int tq_prefill_attention(const void* q, int32_t dtype, int64_t sqb, int64_t sqh,
+                         int64_t sqs, const uint16_t* key_pi_split,
+                         const uint16_t* key_s_eff_f16, const uint8_t* key_codes,
+                         const uint8_t* key_signs, const uint16_t* key_rn,
+                         const uint16_t* key_vn, const uint16_t* key_centroids_f16,
+                         int32_t bits, const uint8_t* val_codes, const uint16_t* val_vn,
+                         const float* val_centroids, int32_t val_bits,
+                         const uint16_t* val_pit_split, int32_t B, int32_t Hq,
+                         int32_t Hkv, int32_t Sq, int32_t Sk, int64_t kv_stride,
+                         int32_t d, float coeff, float scale, int32_t causal,
+                         const void* mask, int32_t mask_dtype, int64_t smb, int64_t smh,
+                         int64_t smq, int64_t smk, void* out, int32_t out_dtype,
+                         void* workspace, int64_t workspace_bytes, void* stream);
+
+/* Workspace bytes of tq_prefill_attention; 0 for shapes it does not take (head dims outside
+ * the supported set, more than 128 query heads per kv head, an empty dimension).  masked:
+ * whether a mask will be passed. */
+int64_t tq_prefill_workspace_size(int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq,
+                                  int32_t Sk, int32_t d, int32_t causal,
+                                  int32_t masked);
+
 /* Compressed-cache append: compress the S new keys and values of each (batch, kv head),
  * k / v [B, H, S, d] (element strides; unit stride on d), into rows [pos, pos + S) of
  * cache planes that hold `capacity` positions per (batch, kv head) -- key_codes

@@ -1,0 +1,227 @@
+"""Attention over expanded key / value tiles (tq_prefill_attention, csrc/tq_dense.hip).
+
+Many query rows per kv head take this path through compressed_attention and
+TurboQuantCache.append_attend.  Reference: the float64 estimator on the device's own planes,
+q_rot rounded to f16 and key centroids / S_eff at f16 as the estimator defines them.
+
+Bars.  The kernel rounds V^ = C_v[c] vn to f16 (relative 2^-11 per element, independent signs)
+and, at head_dim 64 / 128 with equal bits, the softmax weights too, so a row's relative error is
+at most about sqrt(2) 2^-11 / sqrt(3) = 4e-4 (uniform rounding errors); q_rot's own f16 rounding
+can fall either way between the f32 and the f64 rotation, which moves a score by 2^-11 of one
+term in rare cases.  REL = 1e-3 covers both with a factor of two.
+"""
+
+import ctypes
+import math
+
+import pytest
+import torch
+
+from transformers_turboquant import TurboQuantCache
+from turboquant_pytorch import _native, compressed_attention
+from turboquant_pytorch.compressors import TurboQuantCompressorMSE, TurboQuantCompressorV2, _tables
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+REL = 1e-3
+
+
+def _unpack(p, b, d):
+    bits = ((p.unsqueeze(-1) >> torch.arange(8, device=p.device, dtype=torch.uint8)) & 1)
+    bits = bits.reshape(p.shape[0], -1)[:, : d * b].reshape(-1, d, b).long()
+    return (bits << torch.arange(b, device=p.device)).sum(-1)
+
+
+def _reference(q, kc, vc, ck, cv, mask=None, causal=False):
+    B, Hq, Sq, D = q.shape
+    _, Hkv, Sk, _ = ck["shape"]
+    G, n = Hq // Hkv, B * Hkv * Sk
+    pi, se = kc.Pi.double(), _tables(kc, q.device, True).s_eff16.double()
+    codes = _unpack(ck["packed_key_indices"].reshape(n, -1), kc.mse_bits, D)
+    sg = _unpack(ck["packed_qjl_signs"].reshape(n, -1), 1, D).double() * 2 - 1
+    coeff = math.sqrt(math.pi / 2) / D
+    kh = kc.centroids.half().double()[codes] * ck["vec_norms"].reshape(n, 1).double()
+    kh += (sg @ se) * (coeff * ck["residual_norm"].reshape(n, 1).double())
+    vh = vc.centroids.double()[_unpack(cv["packed_indices"].reshape(n, -1), vc.bits, D)]
+    vh = vh * cv["vec_norms"].reshape(n, 1).double()
+    kh, vh = (t.reshape(B, Hkv, Sk, D).repeat_interleave(G, dim=1) for t in (kh, vh))
+    s = ((q.double() @ pi.T).half().double() @ kh.transpose(-2, -1).contiguous()) / math.sqrt(D)
+    if mask is not None:
+        s = s + mask.double().clamp(min=-3e38 / 1.4426950408889634)
+    if causal:
+        i = torch.arange(Sq, device=q.device)[:, None] + (Sk - Sq)
+        s = s.masked_fill(torch.arange(Sk, device=q.device)[None] > i, -math.inf)
+    return ((torch.softmax(s, -1) @ vh) @ vc.Pi.double()).transpose(1, 2)
+
+
+def _make(d, bits, vbits, hq, hkv, sq, sk, dtype=torch.float32, B=2, scale=None, seed=0):
+    g = torch.Generator(device=DEV).manual_seed(seed + d + 7 * sk + sq)
+    r = lambda *s: torch.randn(*s, device=DEV, generator=g)  # noqa: E731
+    kc = TurboQuantCompressorV2(d, bits, seed=42, device=DEV)
+    vc = TurboQuantCompressorMSE(d, vbits, seed=10042, device=DEV)
+    k = r(B, hkv, sk, d)
+    if scale is not None:
+        k = k * scale(sk)
+    return kc, vc, r(B, hq, sq, d).to(dtype), kc.compress(k.to(dtype)), vc.compress(r(B, hkv, sk, d).to(dtype))
+
+
+def _err(got, ref):
+    assert torch.isfinite(got).all()
+    return ((got.double() - ref).norm() / ref.norm()).item()
+
+
+@pytest.mark.parametrize("d,bits,vbits,hq,hkv,sq,sk,causal", [
+    (128, 3, 3, 8, 2, 64, 64, True),       # one block of 256 columns, whole tiles
+    (128, 2, 2, 8, 2, 65, 65, True),       # a second block and a second tile of one row / key
+    (128, 4, 4, 7, 1, 73, 95, True),       # 36 rows of 7 heads per block, 4 columns idle
+    (128, 3, 3, 4, 4, 300, 333, False),    # multi-head, ragged tail tile
+    (128, 3, 3, 32, 8, 40, 3000, True),    # keys split over blocks, merged
+    (128, 3, 2, 16, 2, 33, 1100, True),    # value bits below the key bits (hi + lo weights)
+    (64, 3, 3, 12, 12, 129, 129, True),
+    (64, 4, 4, 4, 2, 700, 1500, False),    # 4-wave blocks, split
+    (64, 2, 1, 4, 2, 70, 31, False),       # fewer keys than a tile
+    (32, 3, 3, 8, 2, 100, 257, False),
+    (40, 2, 2, 4, 4, 130, 600, True),      # 5-byte sign rows: byte loads
+    (80, 3, 3, 8, 2, 65, 530, True),
+    (96, 4, 3, 6, 2, 90, 200, True),
+    (112, 3, 3, 4, 1, 50, 90, False),
+    (160, 3, 3, 4, 2, 66, 66, True),
+    (192, 2, 2, 4, 4, 70, 700, True),
+    (200, 3, 3, 4, 4, 64, 64, False),
+    (224, 3, 3, 4, 4, 64, 100, True),
+    (256, 4, 4, 4, 2, 100, 300, True),
+])
+def test_prefill_shapes(d, bits, vbits, hq, hkv, sq, sk, causal):
+    print("case:", d, bits, vbits, hq, hkv, sq, sk, causal, flush=True)
+    kc, vc, q, ck, cv = _make(d, bits, vbits, hq, hkv, sq, sk)
+    got = compressed_attention(q, kc, vc, ck, cv, causal=causal)
+    assert _err(got, _reference(q, kc, vc, ck, cv, causal=causal)) < REL
+
+
+@pytest.mark.parametrize("d", [64, 80, 128, 256])
+@pytest.mark.parametrize("mdt", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("sk,layout", [(160, "batch"), (161, "batch"), (200, "head"), (96, "strided")])
+def test_prefill_masks(d, mdt, sk, layout):
+    """Additive masks in their own type: broadcast over heads, per head, rows that start off a
+    dword (odd key counts), and a layout that is not contiguous in keys."""
+    print("case:", d, mdt, sk, layout, flush=True)
+    sq, hq, hkv, B = 100, 8, 2, 2
+    kc, vc, q, ck, cv = _make(d, 3, 3, hq, hkv, sq, sk)
+    g = torch.Generator(device=DEV).manual_seed(sk)
+    m = torch.randn(B, hq if layout == "head" else 1, sq, sk, device=DEV, generator=g).to(mdt)
+    m[0, :, :, : sk // 3] = torch.finfo(mdt).min          # left padding
+    m[1, :, 5:9, 40:] = -math.inf
+    if layout == "strided":
+        m = m.transpose(-1, -2).contiguous().transpose(-1, -2)
+    got = compressed_attention(q, kc, vc, ck, cv, attention_mask=m)
+    assert _err(got, _reference(q, kc, vc, ck, cv, mask=m.expand(B, hq, sq, sk))) < REL
+
+
+def test_prefill_rows_without_a_real_key():
+    """A row whose mask is finfo.min everywhere attends all keys equally, as softmax does."""
+    kc, vc, q, ck, cv = _make(128, 3, 3, 8, 2, 70, 100)
+    m = torch.zeros(2, 1, 70, 100, device=DEV)
+    m[0, :, 3] = torch.finfo(torch.float32).min
+    m[1, :, :, 50:] = torch.finfo(torch.float32).min
+    got = compressed_attention(q, kc, vc, ck, cv, attention_mask=m)
+    assert _err(got, _reference(q, kc, vc, ck, cv, mask=m.expand(2, 8, 70, 100))) < REL
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("d", [80, 128])
+def test_prefill_dtypes_and_strides(d, dtype):
+    """Queries of each type, as the transposed view a projection leaves, and with rows that are
+    not 16-byte aligned."""
+    kc, vc, q, ck, cv = _make(d, 3, 3, 8, 2, 70, 140, dtype)
+    ref = _reference(q, kc, vc, ck, cv, causal=True)
+    base = compressed_attention(q, kc, vc, ck, cv, causal=True, out_dtype=torch.float32)
+    assert _err(base, ref) < REL
+    view = q.transpose(1, 2).contiguous().transpose(1, 2)
+    buf = torch.empty(q.numel() + 1, device=DEV, dtype=dtype)[1:]
+    off = buf.copy_(q.reshape(-1)).view(q.shape)
+    for x in (view, off):
+        assert torch.equal(compressed_attention(x, kc, vc, ck, cv, causal=True, out_dtype=torch.float32), base)
+    out = compressed_attention(q, kc, vc, ck, cv, causal=True)
+    assert out.dtype == dtype and torch.equal(out, base.to(dtype))
+
+
+@pytest.mark.parametrize("qs,ks", [(1.0, 1.0), (1e-3, 3e2), (300.0, 1e-2), (1.0, 1e-4)])
+def test_prefill_norm_ranges(qs, ks):
+    """Key norms over five decades inside every tile (the tile's power of two follows its largest)
+    and query norms that keep the scores in softmax's range.  The norm planes are f16, so the
+    largest norm stays below 65504: sqrt(128) * 1.4 (the widest of these rows) * 10 * 3e2 = 4.8e4."""
+    kc, vc, q, ck, cv = _make(128, 3, 3, 8, 2, 64, 320, scale=lambda s: ks * 10 ** torch.linspace(
+        -4, 1, 32, device=DEV).repeat(s // 32)[:, None])
+    got = compressed_attention(q * qs, kc, vc, ck, cv, causal=True)
+    assert _err(got, _reference(q * qs, kc, vc, ck, cv, causal=True)) < REL
+
+
+def test_prefill_chunk_over_cache_planes():
+    """A prompt chunk through TurboQuantCache.append_attend: capacity planes (kv_stride) against
+    the compact planes of one compression, bit for bit, and against the reference."""
+    d, hq, hkv, sk, sq = 128, 8, 2, 700, 150
+    g = torch.Generator(device=DEV).manual_seed(3)
+    k, v, q = (torch.randn(2, h, n, d, device=DEV, generator=g).bfloat16()
+               for h, n in ((hkv, sk), (hkv, sk), (hq, sq)))
+    kc = TurboQuantCompressorV2(d, 3, seed=42, device=DEV)
+    vc = TurboQuantCompressorMSE(d, 3, seed=10042, device=DEV)
+    cache = TurboQuantCache()
+    cache.append(0, kc, vc, k[:, :, : sk - sq], v[:, :, : sk - sq])
+    got = cache.append_attend(0, kc, vc, k[:, :, sk - sq:], v[:, :, sk - sq:], q, causal=True)
+    ck, cv = kc.compress(k), vc.compress(v)
+    assert torch.equal(got, compressed_attention(q, kc, vc, ck, cv, causal=True, out_dtype=torch.float32))
+    assert _err(got, _reference(q, kc, vc, ck, cv, causal=True)) < REL
+
+
+@pytest.mark.parametrize("sq,sk", [(100, 100), (40, 3000)])
+def test_prefill_rounds_over_a_small_workspace(sq, sk):
+    """A workspace of one (batch, kv head) runs them in rounds over the same memory: bit-identical
+    to all at once; one byte less is refused."""
+    d, hq, hkv, B = 128, 32, 8, 1
+    kc, vc, q, ck, cv = _make(d, 3, 3, hq, hkv, sq, sk, B=B)
+    tk, tv = _tables(kc, q.device, True), _tables(vc, q.device, False)
+    lib = _native.lib()
+    full = lib.tq_prefill_workspace_size(B, hq, hkv, sq, sk, d, 1, 0)
+    q_part = 2 * d * d + (B * hq * sq * d * 2 + 255) // 256 * 256  # S_eff fragments and q_rot
+    group = (full - q_part) // (B * hkv)
+    assert (full - q_part) % (B * hkv) == 0
+
+    def run(nbytes):
+        out = torch.zeros(B, sq, hq, d, device=DEV)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=DEV)
+        p = _native.ptr
+        st = lib.tq_prefill_attention(
+            p(q), 0, q.stride(0), q.stride(1), q.stride(2), p(tk.pi_split), p(tk.s_eff16),
+            p(ck["packed_key_indices"]), p(ck["packed_qjl_signs"]), p(ck["residual_norm"]), p(ck["vec_norms"]),
+            p(tk.cent16), 3, p(cv["packed_indices"]), p(cv["vec_norms"]), p(tv.cent32), 3, p(tv.pit_split), B, hq,
+            hkv, sq, sk, 0, d, math.sqrt(math.pi / 2) / d, 1 / math.sqrt(d), 1, None, 0, 0, 0, 0, 0, p(out), 0,
+            p(ws), ctypes.c_int64(nbytes), torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        return st, out
+
+    st, whole = run(full)
+    assert st == 0
+    st, one = run(q_part + group)
+    assert st == 0 and torch.equal(one, whole)
+    assert run(q_part + group - 1)[0] == -1
+    assert torch.equal(whole, compressed_attention(q, kc, vc, ck, cv, causal=True))
+
+
+def test_prefill_under_graph_capture():
+    kc, vc, q, ck, cv = _make(128, 3, 3, 8, 2, 200, 900)
+    ref = compressed_attention(q, kc, vc, ck, cv, causal=True)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        compressed_attention(q, kc, vc, ck, cv, causal=True)
+    torch.cuda.current_stream().wait_stream(s)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = compressed_attention(q, kc, vc, ck, cv, causal=True)
+    for rep in range(4):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref), rep
+        compressed_attention(q * (rep + 2), kc, vc, ck, cv, causal=True)
+        torch.cuda.synchronize()

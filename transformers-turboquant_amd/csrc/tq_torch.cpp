@@ -107,6 +107,22 @@ int64_t kv_rows(int64_t B, int64_t hkv, int64_t sk, int64_t kv_stride) {
   return B * hkv > 0 ? (B * hkv - 1) * stride + sk : 0;
 }
 
+// key planes and the head counts of queries [B, Hq, Sq, D] (sizes read from q)
+void check_keys(const Checker& c, const Tensor& q, const Tensor& codes, const Tensor& signs, const Tensor& rn,
+                const Tensor& vn, const Tensor& cent16, int64_t bits, int64_t hkv, int64_t sk, int64_t kv_stride) {
+  const int64_t B = q.size(0), Hq = q.size(1), D = q.size(3);
+  TORCH_CHECK(bits >= 2 && bits <= 9, c.op, ": key bits must be 2..9, got ", bits);
+  TORCH_CHECK(hkv >= 1 && Hq % hkv == 0, c.op, ": ", Hq, " query heads are not a multiple of ", hkv, " kv heads");
+  TORCH_CHECK(sk >= 0 && (kv_stride == 0 || kv_stride >= sk), c.op, ": kv_stride ", kv_stride,
+              " must be 0 or at least Sk = ", sk);
+  const int64_t rows = kv_rows(B, hkv, sk, kv_stride);
+  c.plane(codes, "packed_key_indices", at::kByte, rows, out_cols(D, bits - 1));
+  c.plane(signs, "packed_qjl_signs", at::kByte, rows, out_cols(D, 1));
+  c.plane(rn, "residual_norm", at::kHalf, rows);
+  c.plane(vn, "vec_norms (keys)", at::kHalf, rows);
+  c.table(cent16, "key centroids", at::kHalf, int64_t{1} << (bits - 1));
+}
+
 // prepared queries and the key planes of tq::scores / tq::attention
 void check_prepared_keys(const Checker& c, const Tensor& q_rot, const Tensor& q_proj, const Tensor& codes,
                          const Tensor& signs, const Tensor& rn, const Tensor& vn, const Tensor& cent16, int64_t bits,
@@ -118,17 +134,7 @@ void check_prepared_keys(const Checker& c, const Tensor& q_rot, const Tensor& q_
   c.same_device(q_proj, "q_proj");
   TORCH_CHECK(q_proj.sizes() == q_rot.sizes(), c.op, ": q_proj ", q_proj.sizes(), " differs from q_rot ",
               q_rot.sizes());
-  const int64_t B = q_rot.size(0), Hq = q_rot.size(1), D = q_rot.size(3);
-  TORCH_CHECK(bits >= 2 && bits <= 9, c.op, ": key bits must be 2..9, got ", bits);
-  TORCH_CHECK(hkv >= 1 && Hq % hkv == 0, c.op, ": ", Hq, " query heads are not a multiple of ", hkv, " kv heads");
-  TORCH_CHECK(sk >= 0 && (kv_stride == 0 || kv_stride >= sk), c.op, ": kv_stride ", kv_stride,
-              " must be 0 or at least Sk = ", sk);
-  const int64_t rows = kv_rows(B, hkv, sk, kv_stride);
-  c.plane(codes, "packed_key_indices", at::kByte, rows, out_cols(D, bits - 1));
-  c.plane(signs, "packed_qjl_signs", at::kByte, rows, out_cols(D, 1));
-  c.plane(rn, "residual_norm", at::kHalf, rows);
-  c.plane(vn, "vec_norms (keys)", at::kHalf, rows);
-  c.table(cent16, "key centroids", at::kHalf, int64_t{1} << (bits - 1));
+  check_keys(c, q_rot, codes, signs, rn, vn, cent16, bits, hkv, sk, kv_stride);
 }
 
 void check_values(const Checker& c, const Tensor& q_rot, const Tensor& vcodes, const Tensor& vvn,
@@ -144,13 +150,23 @@ void check_values(const Checker& c, const Tensor& q_rot, const Tensor& vcodes, c
 }
 
 // the additive mask as a float32 view broadcast to [B, Hq, Sq, Sk] (no copy when it already
-// is float32 on the device)
-Tensor attention_mask(const Checker& c, const c10::optional<Tensor>& mask_in, const Tensor& q_rot, int64_t sk) {
+// is float32 on the device); `own_type`: float16 and bfloat16 masks stay as they are.  `rows`: for
+// kernels that copy whole row segments, a mask that is not contiguous in keys, or whose 16-bit rows
+// start off a dword (odd key counts), is laid out anew before it is broadcast (read element by
+// element instead, a layer of 2 x 32 heads x 2869 rows under such a mask took 2.26 ms; as float32 rows 0.89)
+Tensor attention_mask(const Checker& c, const c10::optional<Tensor>& mask_in, const Tensor& q_rot, int64_t sk,
+                      bool own_type = false, bool rows = false) {
   if (!mask_in.has_value() || !mask_in->defined()) return Tensor();
   Tensor mask = *mask_in;
   TORCH_CHECK(mask.dim() <= 4, c.op, ": the mask must broadcast to [B, Hq, Sq, Sk], got ", mask.sizes());
-  if (mask.device() != q_rot.device() || mask.scalar_type() != at::kFloat) mask = mask.to(q_rot.device(), at::kFloat);
+  const at::ScalarType type = own_type && is_act(mask.scalar_type()) ? mask.scalar_type() : at::kFloat;
+  if (mask.device() != q_rot.device() || mask.scalar_type() != type) mask = mask.to(q_rot.device(), type);
   while (mask.dim() < 4) mask = mask.unsqueeze(0);
+  if (rows && mask.size(3) > 1) {
+    if (mask.stride(3) != 1) mask = mask.contiguous();
+    const bool odd = ((mask.storage_offset() | mask.stride(0) | mask.stride(1) | mask.stride(2)) & 1) != 0;
+    if (mask.scalar_type() != at::kFloat && odd) mask = mask.to(at::kFloat).contiguous();
+  }
   return mask.expand({q_rot.size(0), q_rot.size(1), q_rot.size(2), sk});
 }
 
@@ -546,6 +562,93 @@ Tensor attention(const Tensor& q_rot, const Tensor& q_proj, const Tensor& kcodes
   return out;
 }
 
+// Shapes that tq_prefill_attention takes over from tq_query_prep + tq_attention_fwd_kv.
+bool prefill_route(int64_t B, int64_t Hq, int64_t hkv, int64_t Sq, int64_t sk, int64_t D, int64_t bits,
+                   int64_t val_bits, bool causal, bool masked) {
+  if (B < 1 || Hq < 1 || Sq < 1 || sk < 1 || bits < 2 || bits > 4 || val_bits < 1 || val_bits > 4) return false;
+  if (causal && sk < Sq) return false;
+  const int64_t G = Hq / hkv;
+  if (G > 128 || D < 8 || D > 256 || D % 8 != 0) return false;
+  // Few columns (query rows x group) per kv head over many keys stay on the kernels that read the
+  // packed planes once, split over keys: expanding a key costs about as much as scoring it for 64
+  // columns there (32/8 heads, head_dim 128, 16 rows x 4k keys: 42 us packed, 69 us expanded; 24
+  // rows, past one block of those kernels: 205 us packed, 70 us expanded).  Those kernels split from
+  // 512 keys on and up to 128 columns (64 under a mask or above head_dim 64 without the prefill
+  // kernel); below 512 keys expanded is level at 64 columns and ahead from there.
+  const bool own = (D == 64 || D == 128) && bits == val_bits;  // the prefill kernel's shapes
+  const bool two_blocks = own ? !masked : D <= 64;
+  // Under a mask the prefill kernel's 64-column blocks are level while they leave the chip's 512
+  // block slots partly idle (32/32 heads, 500 rows: 82 us packed, 86 us expanded; 4 x 12 heads, 1000
+  // rows: 109 and 94 us)
+  if (own && masked && sk <= 1024 && B * hkv * ((G * Sq + 63) / 64) <= 512) return false;
+  const int64_t split_cols = two_blocks ? 128 : 64;
+  return sk >= 512 ? G * Sq > split_cols : G * Sq >= 64;
+}
+
+// Attention of raw queries: the checks, and the [B, Sq, Hq, D] output
+Tensor attend_meta(const Tensor& q, const Tensor& pi_split, const Tensor& s_eff16, const Tensor& kcodes,
+                   const Tensor& ksigns, const Tensor& krn, const Tensor& kvn, const Tensor& kcent16, int64_t bits,
+                   const Tensor& vcodes, const Tensor& vvn, const Tensor& vcent32, int64_t val_bits,
+                   const Tensor& vpit, int64_t hkv, int64_t sk, int64_t kv_stride, double coeff, double scale,
+                   bool causal, const c10::optional<Tensor>& mask_in, at::ScalarType out_dtype, int64_t workspace) {
+  const Checker c{"tq::attend", q.device()};
+  TORCH_CHECK(q.dim() == 4, c.op, ": expected [B, Hq, Sq, D] queries");
+  TORCH_CHECK(workspace >= 0 && workspace <= 2, c.op, ": workspace mode must be 0, 1 or 2");
+  TORCH_CHECK(is_act(out_dtype), c.op, ": out_dtype must be float32, float16 or bfloat16");
+  const int64_t D = q.size(3);
+  c.table(pi_split, "split Pi", at::kHalf, 2 * D * D);
+  c.table(s_eff16, "f16 S_eff", at::kHalf, D * D);
+  check_keys(c, q, kcodes, ksigns, krn, kvn, kcent16, bits, hkv, sk, kv_stride);
+  check_values(c, q, vcodes, vvn, vcent32, val_bits, vpit, hkv, sk, kv_stride);
+  attention_mask(c, mask_in, q, sk, true);  // broadcastable to [B, Hq, Sq, Sk]
+  return at::empty({q.size(0), q.size(2), q.size(1), D}, q.options().dtype(out_dtype));
+}
+
+// Attention of raw queries over packed planes: tq_prefill_attention where it is the faster
+// choice and torch may allocate its workspace (mode 1), otherwise query_prep and attention.
+Tensor attend(const Tensor& q_in, const Tensor& pi_split, const Tensor& s_eff16, const Tensor& kcodes,
+              const Tensor& ksigns, const Tensor& krn, const Tensor& kvn, const Tensor& kcent16, int64_t bits,
+              const Tensor& vcodes, const Tensor& vvn, const Tensor& vcent32, int64_t val_bits, const Tensor& vpit,
+              int64_t hkv, int64_t sk, int64_t kv_stride, double coeff, double scale, bool causal,
+              const c10::optional<Tensor>& mask_in, at::ScalarType out_dtype, int64_t workspace) {
+  const bool route = workspace == 1 && q_in.dim() == 4 && hkv >= 1 && q_in.size(1) % hkv == 0 &&
+                     prefill_route(q_in.size(0), q_in.size(1), hkv, q_in.size(2), sk, q_in.size(3), bits, val_bits,
+                                   causal, mask_in.has_value() && mask_in->defined());
+  if (!route) {
+    auto qp = query_prep(q_in, pi_split, s_eff16);
+    return attention(std::get<0>(qp), std::get<1>(qp), kcodes, ksigns, krn, kvn, kcent16, bits, vcodes, vvn, vcent32,
+                     val_bits, vpit, hkv, sk, kv_stride, coeff, scale, causal, mask_in, out_dtype, workspace);
+  }
+  Tensor out = attend_meta(q_in, pi_split, s_eff16, kcodes, ksigns, krn, kvn, kcent16, bits, vcodes, vvn, vcent32,
+                           val_bits, vpit, hkv, sk, kv_stride, coeff, scale, causal, mask_in, out_dtype, workspace);
+  const Checker c{"tq::attend", q_in.device()};
+  const c10::DeviceGuard g(q_in.device());
+  Tensor q = activation(q_in);
+  const int64_t B = q.size(0), Hq = q.size(1), Sq = q.size(2), D = q.size(3);
+  Tensor mask = attention_mask(c, mask_in, q, sk, true, true);
+  int64_t ms[4] = {0, 0, 0, 0};
+  if (mask.defined())
+    for (int i = 0; i < 4; ++i) ms[i] = mask.stride(i);
+  const int64_t bytes = tq_prefill_workspace_size(static_cast<int32_t>(B), static_cast<int32_t>(Hq),
+                                                  static_cast<int32_t>(hkv), static_cast<int32_t>(Sq),
+                                                  static_cast<int32_t>(sk), static_cast<int32_t>(D), causal ? 1 : 0,
+                                                  mask.defined() ? 1 : 0);
+  Tensor ws = at::empty({bytes}, q.options().dtype(at::kByte));
+  check_status(tq_prefill_attention(
+                   q.data_ptr(), dtype_code(q.scalar_type()), q.stride(0), q.stride(1), q.stride(2),
+                   ptr<uint16_t>(pi_split), ptr<uint16_t>(s_eff16), ptr<uint8_t>(kcodes), ptr<uint8_t>(ksigns),
+                   ptr<uint16_t>(krn), ptr<uint16_t>(kvn), ptr<uint16_t>(kcent16), static_cast<int32_t>(bits),
+                   ptr<uint8_t>(vcodes), ptr<uint16_t>(vvn), ptr<float>(vcent32), static_cast<int32_t>(val_bits),
+                   ptr<uint16_t>(vpit), static_cast<int32_t>(B), static_cast<int32_t>(Hq), static_cast<int32_t>(hkv),
+                   static_cast<int32_t>(Sq), static_cast<int32_t>(sk), kv_stride, static_cast<int32_t>(D),
+                   static_cast<float>(coeff), static_cast<float>(scale), causal ? 1 : 0,
+                   mask.defined() ? mask.data_ptr() : nullptr,
+                   mask.defined() ? dtype_code(mask.scalar_type()) : static_cast<int32_t>(TQ_F32), ms[0], ms[1], ms[2],
+                   ms[3], out.data_ptr(), dtype_code(out_dtype), ws.data_ptr(), bytes, stream_of(out)),
+               "compressed_attention");
+  return out;
+}
+
 // A cached decode step in one call: cache_append (the new keys / values into the capacity
 // planes at row pos, the new queries prepared in the same launch), then attention over the
 // planes' first pos + S rows.  The same two operators back to back, without the second
@@ -558,6 +661,18 @@ Tensor cache_attend(const Tensor& k, const Tensor& v, const Tensor& q, const Ten
                     const Tensor& vvn, int64_t pos, const Tensor& kcent16, const Tensor& vcent32, const Tensor& vpit,
                     double coeff, double scale, bool causal, const c10::optional<Tensor>& mask,
                     at::ScalarType out_dtype, int64_t workspace) {
+  if (workspace == 1 && k.dim() == 4 && q.dim() == 4 && k.size(1) >= 1 && q.size(1) % k.size(1) == 0 &&
+      q.size(0) == k.size(0) && q.size(2) == k.size(2) && q.size(3) == k.size(3) && q.device() == k.device() &&
+      prefill_route(q.size(0), q.size(1), k.size(1), q.size(2), pos + k.size(2), q.size(3), key_code_bits + 1,
+                    val_bits, causal, mask.has_value() && mask->defined())) {
+    // a prompt chunk: the new rows appended, then attention from the raw queries (taken in k's
+    // type, as cache_append does)
+    cache_append(k, v, c10::nullopt, kpi, kseff, kcent, kbounds, key_code_bits, vpi, vbounds, val_bits, kseff16,
+                 kcodes, ksigns, krn, kvn, vcodes, vvn, pos);
+    return attend(is_act(k.scalar_type()) ? q.to(k.scalar_type()) : q.to(at::kFloat), kpi, kseff16, kcodes, ksigns,
+                  krn, kvn, kcent16, key_code_bits + 1, vcodes, vvn, vcent32, val_bits, vpit, k.size(1),
+                  pos + k.size(2), kvn.size(-1), coeff, scale, causal, mask, out_dtype, workspace);
+  }
   auto qp = cache_append(k, v, q, kpi, kseff, kcent, kbounds, key_code_bits, vpi, vbounds, val_bits, kseff16, kcodes,
                          ksigns, krn, kvn, vcodes, vvn, pos);
   return attention(std::get<0>(qp), std::get<1>(qp), kcodes, ksigns, krn, kvn, kcent16, key_code_bits + 1, vcodes, vvn,
@@ -609,6 +724,10 @@ TORCH_LIBRARY(tq, m) {
         "Tensor kcent, int bits, Tensor vcodes, Tensor vvn, Tensor vcent, int val_bits, Tensor vpit, int hkv, "
         "int sk, int kv_stride, float coeff, float scale, bool causal, Tensor? mask, ScalarType out_dtype, "
         "int workspace) -> Tensor");
+  m.def("attend(Tensor q, Tensor pi_split, Tensor s_eff, Tensor kcodes, Tensor ksigns, Tensor krn, Tensor kvn, "
+        "Tensor kcent, int bits, Tensor vcodes, Tensor vvn, Tensor vcent, int val_bits, Tensor vpit, int hkv, "
+        "int sk, int kv_stride, float coeff, float scale, bool causal, Tensor? mask, ScalarType out_dtype, "
+        "int workspace) -> Tensor");
   m.def("cache_attend(Tensor k, Tensor v, Tensor q, Tensor kpi, Tensor kseff, Tensor kcent, Tensor kbounds, "
         "int key_code_bits, Tensor vpi, Tensor vbounds, int val_bits, Tensor kseff16, Tensor(a!) kcodes, "
         "Tensor(b!) ksigns, Tensor(c!) krn, Tensor(d!) kvn, Tensor(e!) vcodes, Tensor(f!) vvn, int pos, "
@@ -629,6 +748,7 @@ TORCH_LIBRARY_IMPL(tq, CUDA, m) {
   m.impl("cache_append", &cache_append);
   m.impl("scores", &scores);
   m.impl("attention", &attention);
+  m.impl("attend", &attend);
   m.impl("cache_attend", &cache_attend);
 }
 
@@ -645,5 +765,6 @@ TORCH_LIBRARY_IMPL(tq, Meta, m) {
   m.impl("cache_append", &cache_append_meta);
   m.impl("scores", &scores_meta);
   m.impl("attention", &attention_meta);
+  m.impl("attend", &attend_meta);
   m.impl("cache_attend", &cache_attend_meta);
 }

@@ -177,14 +177,13 @@ class TurboQuantCacheLayer(CacheLayerMixin):
         tk, tv, need = self._gpu_room(key_compressor, val_compressor, k)
         if out_dtype not in (torch.float32, torch.float16, torch.bfloat16):
             out_dtype = torch.float32
-        mask = attention_mask.to(k.device, torch.float32) if attention_mask is not None else None
         out = ops().cache_attend(
             k, v, q, tk.pi_split, tk.seff_split, tk.cent32, tk.bounds32, key_compressor.mse_bits, tv.pi_split,
             tv.bounds32, val_compressor.bits, tk.s_eff16, self.kp["packed_key_indices"], self.kp["packed_qjl_signs"],
             self.kp["residual_norm"], self.kp["vec_norms"], self.vp["packed_indices"], self.vp["vec_norms"],
             self.length, tk.cent16, tv.cent32, tv.pit_split,
             float(math.sqrt(math.pi / 2) / key_compressor.S.shape[0]),
-            float(scale if scale is not None else 1.0 / math.sqrt(D)), bool(causal), mask, out_dtype, 1)
+            float(scale if scale is not None else 1.0 / math.sqrt(D)), bool(causal), attention_mask, out_dtype, 1)
         self.length = need
         return out
 
