@@ -254,6 +254,22 @@ int64_t tq_prefill_workspace_size(int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq
                                   int32_t Sk, int32_t d, int32_t causal,
                                   int32_t masked);
 
+/* Materialised scores (as tq_attention_scores_kv) for many query rows, from raw queries and
+ * keys expanded as in tq_prefill_attention: out f32 [B, Hq, Sq, Sk].  Fewer than 2^24 keys.
+ * Replaces compressors.py:178-200, kernels/attention.py:274-372. */
+int tq_prefill_scores(const void* q, int32_t dtype, int64_t sqb, int64_t sqh, int64_t sqs,
+                      const uint16_t* key_pi_split, const uint16_t* key_s_eff_f16,
+                      const uint8_t* key_codes, const uint8_t* key_signs,
+                      const uint16_t* key_rn, const uint16_t* key_vn,
+                      const uint16_t* key_centroids_f16, int32_t bits, int32_t B,
+                      int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Sk, int64_t kv_stride,
+                      int32_t d, float coeff, float* out, void* workspace,
+                      int64_t workspace_bytes, void* stream);
+
+/* Workspace bytes of tq_prefill_scores (0: shape not taken). */
+int64_t tq_prefill_scores_workspace_size(int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq,
+                                         int32_t Sk, int32_t d);
+
 /* Compressed-cache append: compress the S new keys and values of each (batch, kv head),
  * k / v [B, H, S, d] (element strides; unit stride on d), into rows [pos, pos + S) of
  * cache planes that hold `capacity` positions per (batch, kv head) -- key_codes

@@ -225,3 +225,53 @@ def test_prefill_under_graph_capture():
         assert torch.equal(out, ref), rep
         compressed_attention(q * (rep + 2), kc, vc, ck, cv, causal=True)
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("d,bits,hq,hkv,sq,sk,dtype", [
+    (128, 3, 8, 2, 33, 64, torch.float32),       # a second row chunk of one row, whole key tiles
+    (128, 2, 4, 4, 130, 1, torch.bfloat16),      # one key
+    (128, 4, 7, 1, 50, 333, torch.float16),      # ragged tail, blocks over several heads
+    (128, 3, 16, 2, 64, 3001, torch.float32),    # key ranges split over blocks
+    (64, 3, 12, 12, 129, 129, torch.float32),
+    (32, 2, 8, 2, 65, 100, torch.float32),
+    (40, 3, 4, 2, 70, 95, torch.bfloat16),       # byte loads of the packed rows
+    (80, 4, 4, 1, 40, 200, torch.float32),
+    (160, 3, 4, 2, 70, 70, torch.float32),
+    (192, 3, 4, 4, 130, 50, torch.float32),
+    (256, 2, 4, 2, 66, 161, torch.float16),
+])
+def test_expanded_scores(d, bits, hq, hkv, sq, sk, dtype):
+    """Materialised scores: f32 sums over q_rot (f16) and keys at f32 grade.  The reference rounds
+    the f64 rotation to f16; an entry whose rounding falls the other way in the kernel's f32
+    rotation (about 2^-11 of them) moves a score by 2^-11 of one of d terms, a relative error of
+    about 2^-11 sqrt(2^-11) = 1e-5 over a matrix of scores; the bar is twice that.  Rows past a
+    head's end or keys past Sk must not be written: the output is the whole buffer, filled with a
+    marker by a larger allocation around it."""
+    print("case:", d, bits, hq, hkv, sq, sk, dtype, flush=True)
+    kc, _, q, ck, _ = _make(d, bits, bits, hq, hkv, sq, sk, dtype)
+    got = kc.asymmetric_attention_scores(q, ck)
+    B, G, n = 2, hq // hkv, 2 * hkv * sk
+    pi, se = kc.Pi.double(), _tables(kc, q.device, True).s_eff16.double()
+    sg = _unpack(ck["packed_qjl_signs"].reshape(n, -1), 1, d).double() * 2 - 1
+    kh = kc.centroids.half().double()[_unpack(ck["packed_key_indices"].reshape(n, -1), kc.mse_bits, d)]
+    kh = kh * ck["vec_norms"].reshape(n, 1).double()
+    kh += (sg @ se) * (math.sqrt(math.pi / 2) / d * ck["residual_norm"].reshape(n, 1).double())
+    kh = kh.reshape(B, hkv, sk, d).repeat_interleave(G, dim=1)
+    ref = (q.double() @ pi.T).half().double() @ kh.transpose(-2, -1).contiguous()
+    assert got.shape == ref.shape and got.dtype == torch.float32
+    assert _err(got, ref) < 2e-5
+
+    # the C entry point writes exactly [B, Hq, Sq, Sk]
+    t = _tables(kc, q.device, True)
+    guard, lib, p = 4096, _native.lib(), _native.ptr
+    buf = torch.full((ref.numel() + 2 * guard,), 7.0, device=DEV)
+    nb = lib.tq_prefill_scores_workspace_size(B, hq, hkv, sq, sk, d)
+    ws = torch.empty(nb, dtype=torch.uint8, device=DEV)
+    st = lib.tq_prefill_scores(
+        p(q), {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}[dtype], q.stride(0), q.stride(1), q.stride(2),
+        p(t.pi_split), p(t.s_eff16), p(ck["packed_key_indices"]), p(ck["packed_qjl_signs"]), p(ck["residual_norm"]),
+        p(ck["vec_norms"]), p(t.cent16), bits, B, hq, hkv, sq, sk, 0, d, math.sqrt(math.pi / 2) / d,
+        p(buf) + 4 * guard, p(ws), ctypes.c_int64(nb), torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert st == 0 and (buf[:guard] == 7).all() and (buf[-guard:] == 7).all()
+    assert torch.equal(buf[guard:-guard].view(ref.shape), got)

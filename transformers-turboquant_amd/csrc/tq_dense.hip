@@ -61,8 +61,8 @@ __device__ __forceinline__ half8 mat8(const uint16_t* m, int i, int j, int d) {
 }
 
 constexpr int kDenseKeys = 32;  // keys per tile
-template <int DP>
-constexpr int dense_rec() { return 3 * DP * 64; }  // bytes of a tile record
+template <int DP, bool VALS = true>
+constexpr int dense_rec() { return (VALS ? 3 : 2) * DP * 64; }  // bytes of a tile record; keys only without VALS
 
 // ---------------------------------------------------------------- query rotation
 // q_rot = f16(q Pi^T) of q[B, Hq, Sq, d] (element strides), rows in (b, h, s) order.
@@ -259,17 +259,17 @@ __device__ __forceinline__ Field32 load_field(const uint8_t* row, int blk, int b
 // One wave per 32-dim block; blocks walk the tiles.  Lane (key n, half h) of wave w ends with
 // dims 32w + 16s + 8h + 0..7 (s = 0, 1) of its key: exactly its 16 bytes of k^ fragments 2w + s.
 // V^ is transposed through a wave-private LDS tile.
-template <int DP, bool DW>
+template <int DP, bool DW, bool VALS>
 __global__ void __launch_bounds__(2 * DP) dense_expand_kernel(ExpandArgs a) {
   constexpr int KS = DP / 16, NW = DP / 32;
   constexpr int VP = 36;  // halves per row of the V^ transposition tile
   __shared__ float s_kc[8], s_vc[16];
   __shared__ float s_bound[NW];
-  __shared__ __attribute__((aligned(16))) _Float16 s_v[NW][32 * VP];
+  __shared__ __attribute__((aligned(16))) _Float16 s_v[VALS ? NW : 1][32 * VP];
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 31, h = lane >> 5, d = a.d;
   if (tid < 8) s_kc[tid] = tid < (1 << a.kb) ? h2f(a.kcent[tid]) : 0.f;
-  if (tid >= 16 && tid < 32) s_vc[tid - 16] = tid - 16 < (1 << a.vb) ? a.vcent[tid - 16] : 0.f;
+  if (VALS && tid >= 16 && tid < 32) s_vc[tid - 16] = tid - 16 < (1 << a.vb) ? a.vcent[tid - 16] : 0.f;
 
   half8 sf[KS];      // S_eff^T rows of this wave's dims
   float asum = 0.f;  // sum over S_eff's rows of |S_eff[., dim]|: bounds |S_eff^T s|
@@ -307,10 +307,10 @@ __global__ void __launch_bounds__(2 * DP) dense_expand_kernel(ExpandArgs a) {
 #pragma unroll
     for (int i = 0; i < NW; ++i) r.sw[i] = load_field<DW>(a.ksigns + row * sc, i, 1, d).w[0];
     r.kf = load_field<DW>(a.kcodes + row * kc, w, a.kb, d);
-    r.vf = load_field<DW>(a.vcodes + row * vc, w, a.vb, d);
+    if constexpr (VALS) r.vf = load_field<DW>(a.vcodes + row * vc, w, a.vb, d);
     r.vn = a.kvn[row];
     r.rn = a.krn[row];
-    r.vvn = a.vvn[row];
+    if constexpr (VALS) r.vvn = a.vvn[row];
     return r;
   };
   Raw nx;
@@ -320,8 +320,7 @@ __global__ void __launch_bounds__(2 * DP) dense_expand_kernel(ExpandArgs a) {
     if (T + gridDim.x < a.total) nx = fetch(T + gridDim.x);
     // keys past Sk have zero norms: k^ and V^ zero
     const float vn = r.ok ? h2f(r.vn) : 0.f, rn = r.ok ? a.coeff * h2f(r.rn) : 0.f;
-    const float vvn = r.ok ? h2f(r.vvn) : 0.f;
-    const Field32 &kf = r.kf, &vf = r.vf;
+    const Field32& kf = r.kf;
     // S_eff^T s: the sign bits as +-1 halves (a clear bit sets the half's sign bit).  Of a byte's
     // clear bits, y holds the even ones from bit 9 and the odd ones from bit 25 on, so that one
     // shift brings each pair to bits 15 and 31
@@ -340,7 +339,7 @@ __global__ void __launch_bounds__(2 * DP) dense_expand_kernel(ExpandArgs a) {
     const float bound = wave_max(vn) * cmax + wave_max(fabsf(rn)) * smax;
     const float up = qproj_split_scale(bound);
     if (tid == 0) a.tfac[T] = 1.f / up;
-    uint8_t* rec = a.tiles + T * dense_rec<DP>();
+    uint8_t* rec = a.tiles + T * dense_rec<DP, VALS>();
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       const bool real = 32 * w + 16 * s + 8 * h < d;  // this lane's 8 dims
@@ -356,29 +355,36 @@ __global__ void __launch_bounds__(2 * DP) dense_expand_kernel(ExpandArgs a) {
       }
       *reinterpret_cast<half8*>(rec + (2 * w + s) * 1024 + lane * 16) = hi;
       *reinterpret_cast<half8*>(rec + (KS + 2 * w + s) * 1024 + lane * 16) = lo;
+    }
+    if constexpr (VALS) {
       // V^ into row perm32 of the block
-      const uint32_t cv = vf.codes8(2 * s + h, a.vb);
+      const float vvn = r.ok ? h2f(r.vvn) : 0.f;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float v = real ? s_vc[(cv >> (a.vb * e)) & vm] * vvn : 0.f;
-        s_v[w][perm32(16 * s + 8 * h + e) * VP + n] = static_cast<_Float16>(v);
+      for (int s = 0; s < 2; ++s) {
+        const bool real = 32 * w + 16 * s + 8 * h < d;
+        const uint32_t cv = r.vf.codes8(2 * s + h, a.vb);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float v = real ? s_vc[(cv >> (a.vb * e)) & vm] * vvn : 0.f;
+          s_v[w][perm32(16 * s + 8 * h + e) * VP + n] = static_cast<_Float16>(v);
+        }
       }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    // fragment 2w + s of V^: row n, keys 16s + 4h + 0..3 and 16s + 8 + 4h + 0..3, the key order
-    // of the accumulator registers 8s..8s+7 that become the P operand
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      // fragment 2w + s of V^: row n, keys 16s + 4h + 0..3 and 16s + 8 + 4h + 0..3, the key order
+      // of the accumulator registers 8s..8s+7 that become the P operand
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const _Float16* p = &s_v[w][n * VP + 16 * s + 4 * h];
-      const half4 x = *reinterpret_cast<const half4*>(p), y = *reinterpret_cast<const half4*>(p + 8);
-      *reinterpret_cast<half8*>(rec + (2 * KS + 2 * w + s) * 1024 + lane * 16) =
-          half8{x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+      for (int s = 0; s < 2; ++s) {
+        const _Float16* p = &s_v[w][n * VP + 16 * s + 4 * h];
+        const half4 x = *reinterpret_cast<const half4*>(p), y = *reinterpret_cast<const half4*>(p + 8);
+        *reinterpret_cast<half8*>(rec + (2 * KS + 2 * w + s) * 1024 + lane * 16) =
+            half8{x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
 }
 
@@ -1028,6 +1034,110 @@ __global__ void __launch_bounds__(2 * DP) dense_merge_kernel(DenseArgs a, int nw
   }
 }
 
+// ---------------------------------------------------------------- materialised scores
+struct DenseScoreArgs {
+  const uint16_t* q_rot;
+  const uint8_t* tiles;  // keys only
+  const float* tfac;
+  int Hq, Hkv, Sq, Sk, d, G, rchunks, nbh, ntile, nblk, cpt;  // rchunks: 32-row chunks of a head
+  int64_t bh0;
+  float* out;  // [B, Hq, Sq, Sk]
+};
+
+// A wave owns 32 query rows of one head (MFMA rows) and walks its block's key tiles (MFMA columns):
+// accumulator register i of lane (key n, h) is row 8 (i / 4) + 4 h + i % 4, so that every store
+// writes 32 consecutive keys of two rows, whole 128-byte lines.  Blocks of 4 waves take
+// consecutive (head, row chunk)s of one kv head and a range of its tiles; records (16 KiB at
+// head_dim 128) reach LDS as in dense_attn_kernel.  Bound by the 4 bytes written per score: 32 heads
+// x 2048 x 2048 take 129 us (4.2 TB/s written; the tiled kernel took 322).  LINES: output rows are
+// whole 128-byte lines, stored past the L2; rows that are not (Sk not a multiple of 32) leave half
+// lines for the L2 to join (32 x 1000 x 1000, whole call: 113 us past it, 76 through it).
+template <int DP, bool LINES>
+__global__ void __launch_bounds__(256) dense_scores_kernel(DenseScoreArgs a) {
+  constexpr int KS = DP / 16, REC = dense_rec<DP, false>(), NF = REC / 1024, CPW = (NF + 3) / 4;
+  constexpr int NS = 3;  // 48 KiB at head_dim 128: three blocks per compute unit
+  __shared__ __attribute__((aligned(16))) uint8_t ring[NS * REC];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 31, h = lane >> 5;
+  const uint32_t bid = blockIdx.x / static_cast<uint32_t>(a.nbh);
+  const int bhi = static_cast<int>(blockIdx.x - bid * a.nbh);
+  const int rb = static_cast<int>(bid % static_cast<uint32_t>(a.nblk)), split = static_cast<int>(bid / static_cast<uint32_t>(a.nblk));
+  const uint32_t bh = static_cast<uint32_t>(a.bh0 + bhi);
+  const int hkv = static_cast<int>(bh % static_cast<uint32_t>(a.Hkv));
+  const int64_t b = bh / static_cast<uint32_t>(a.Hkv);
+  const int tb = split * a.cpt, te = min(a.ntile, tb + a.cpt);
+  if (tb >= te) return;
+  const int task = rb * 4 + wave;  // (head of the group, row chunk)
+  const bool live = task < a.G * a.rchunks;
+  const int gi = live ? task / a.rchunks : 0, r0 = live ? (task - gi * a.rchunks) * 32 : 0;
+  const int hq = hkv * a.G + gi, rows = min(32, a.Sq - r0);
+  const int64_t row0 = (b * a.Hq + hq) * a.Sq + r0;
+  half8 qf[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    const int d0 = 16 * ks + 8 * h;
+    const bool real = n < rows && d0 < a.d;
+    const half8 v = *reinterpret_cast<const half8*>(a.q_rot + (row0 + (n < rows ? n : 0)) * a.d + (real ? d0 : 0));
+    qf[ks] = real ? v : half8{};
+  }
+  // rows past the head's end are dropped by the store's range check
+  const rsrc_t ro = make_rsrc(a.out + row0 * a.Sk, live ? static_cast<uint32_t>(rows) * a.Sk * 4 : 0);
+  const float* tfac = a.tfac + static_cast<int64_t>(bhi) * a.ntile;
+  float fv = 0.f;
+  auto factors = [&](int t) __attribute__((always_inline)) {  // of tiles t .. t + 63
+    fv = tfac[min(t + lane, te - 1)];
+    wait_vm0_visible();
+  };
+  uint64_t src = reinterpret_cast<uint64_t>(a.tiles) + (static_cast<uint64_t>(bhi) * a.ntile + tb) * REC;
+  int left = te - tb;
+  const uint32_t ring_lds = lds_offset(ring);
+  uint32_t dst = ring_lds;
+  auto issue = [&]() __attribute__((always_inline)) {
+    const i32x4 r{static_cast<int>(static_cast<uint32_t>(src)), static_cast<int>(static_cast<uint32_t>(src >> 32) & 0xffffu),
+                  REC, 0x00020000};
+#pragma unroll
+    for (int i = 0; i < CPW; ++i) {
+      const int f = NF % 4 == 0 ? wave + 4 * i : min(wave + 4 * i, NF - 1);
+      dma16_cached(r, dst + f * 1024, f * 1024 + lane * 16);
+    }
+    if (--left > 0) src += REC;
+    dst = dst + REC == ring_lds + NS * REC ? ring_lds : dst + REC;
+  };
+  factors(tb);  // and waits for q
+#pragma unroll
+  for (int i = 0; i < NS - 1; ++i) issue();
+  const uint8_t* rec = ring + lane * 16;
+  for (int t = tb; t < te; ++t) {
+    if (t != tb && ((t - tb) & 63) == 0) factors(t);
+    // tile t's copies have landed: after them come NS - 2 records and, once the ring has gone round,
+    // the 16 stores of each of the last NS - 1 tiles, which need not be waited for
+    if (t - tb >= NS - 1) wait_vm<(NS - 2) * CPW + 16 * (NS - 1)>();
+    else wait_vm<(NS - 2) * CPW>();
+    wait_lds();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    issue();
+    float16v s = zero16();
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      s = mfma32x32x16(qf[ks], *reinterpret_cast<const half8*>(rec + ks * 1024), s);
+      s = mfma32x32x16(qf[ks], *reinterpret_cast<const half8*>(rec + (KS + ks) * 1024), s);
+    }
+    const float f = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, fv), (t - tb) & 63));
+    const int key = t * kDenseKeys + n;
+    // the range check covers the lane offset: it carries the row, and keys past Sk start out of range
+    // (Sk < 2^24: neither wraps)
+    const uint32_t at = key < a.Sk ? static_cast<uint32_t>(4 * h * a.Sk + key) * 4 : kOutOfRange;
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, s[i] * f), ro,
+                                            at + static_cast<uint32_t>((8 * (i >> 2) + (i & 3)) * a.Sk) * 4, 0,
+                                            LINES ? kStream : 0);
+    rec = rec + REC == ring + NS * REC + lane * 16 ? ring + lane * 16 : rec + REC;
+  }
+  wait_vm<0>();  // no copy outlives the block
+}
+
 // ---------------------------------------------------------------- host
 struct DensePlan {
   int NW = 0, QT = 0, nqb = 0, ntile = 0, nsplit = 1, cpt = 0;
@@ -1134,6 +1244,46 @@ static int64_t dense_q_bytes(int B, int Hq, int Sq, int d) {
   return 2 * DP * DP + (static_cast<int64_t>(B) * Hq * Sq * d * 2 + 255) / 256 * 256;
 }
 
+// workspace of one (batch, kv head)'s expanded keys and tile factors
+static int64_t score_group_bytes(int Sk, int d) {
+  const int64_t nt = (Sk + kDenseKeys - 1) / kDenseKeys;
+  return nt * (2 * pad_dim(d) * 64) + (nt * 4 + 15) / 16 * 16;
+}
+
+// q_rot, and S_eff's fragments for the expansion
+static void launch_rotate(const void* q, int dtype, int B, int Hq, int Sq, int d, int64_t sqb, int64_t sqh, int64_t sqs,
+                          const uint16_t* key_pi_split, const uint16_t* key_s_eff_f16, uint16_t* q_rot,
+                          uint16_t* seff_frag, int cus, hipStream_t s) {
+  const int DP = pad_dim(d);
+  RotArgs r{};
+    r.q = q; r.n = static_cast<int64_t>(B) * Hq * Sq; r.sqb = sqb; r.sqh = sqh; r.sqs = sqs;
+    r.Hq = Hq; r.Sq = Sq; r.d = d; r.pi = key_pi_split; r.seff = key_s_eff_f16;
+    r.q_rot = q_rot; r.seff_frag = seff_frag;
+    const int64_t es = dtype == TQ_F32 ? 4 : 2;
+    r.vec = reinterpret_cast<uintptr_t>(q) % 16 == 0 && (sqb * es) % 16 == 0 && (sqh * es) % 16 == 0 &&
+            (sqs * es) % 16 == 0;
+    r.blocks = static_cast<int>(std::min<int64_t>((r.n + 255) / 256, 2LL * cus));
+    const unsigned gx = r.blocks + 4;
+#define TQ_ROT_CASE(DD)                                                                     \
+  case DD: {                                                                                \
+    const dim3 g(gx, (DD / 32 + rot_blocks<DD>() - 1) / rot_blocks<DD>());                  \
+    if (dtype == TQ_F32) dense_rotate_kernel<DD, TQ_F32><<<g, 512, 0, s>>>(r);              \
+    else if (dtype == TQ_F16) dense_rotate_kernel<DD, TQ_F16><<<g, 512, 0, s>>>(r);         \
+    else dense_rotate_kernel<DD, TQ_BF16><<<g, 512, 0, s>>>(r);                             \
+  } break;
+    switch (DP) {
+      TQ_ROT_CASE(32)
+      TQ_ROT_CASE(64)
+      TQ_ROT_CASE(96)
+      TQ_ROT_CASE(128)
+      TQ_ROT_CASE(160)
+      TQ_ROT_CASE(192)
+      TQ_ROT_CASE(224)
+      TQ_ROT_CASE(256)
+    }
+#undef TQ_ROT_CASE
+}
+
 extern "C" {
 
 int64_t tq_prefill_workspace_size(int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Sk, int32_t d,
@@ -1195,35 +1345,7 @@ int tq_prefill_attention(const void* q, int32_t dtype, int64_t sqb, int64_t sqh,
 
   uint16_t* seff_frag = static_cast<uint16_t*>(workspace);
   uint16_t* q_rot = seff_frag + static_cast<int64_t>(DP) * DP;
-  {
-    RotArgs r{};
-    r.q = q; r.n = static_cast<int64_t>(B) * Hq * Sq; r.sqb = sqb; r.sqh = sqh; r.sqs = sqs;
-    r.Hq = Hq; r.Sq = Sq; r.d = d; r.pi = key_pi_split; r.seff = key_s_eff_f16;
-    r.q_rot = q_rot; r.seff_frag = seff_frag;
-    const int64_t es = dtype == TQ_F32 ? 4 : 2;
-    r.vec = reinterpret_cast<uintptr_t>(q) % 16 == 0 && (sqb * es) % 16 == 0 && (sqh * es) % 16 == 0 &&
-            (sqs * es) % 16 == 0;
-    r.blocks = static_cast<int>(std::min<int64_t>((r.n + 255) / 256, 2LL * cus));
-    const unsigned gx = r.blocks + 4;
-#define TQ_ROT_CASE(DD)                                                                     \
-  case DD: {                                                                                \
-    const dim3 g(gx, (DD / 32 + rot_blocks<DD>() - 1) / rot_blocks<DD>());                  \
-    if (dtype == TQ_F32) dense_rotate_kernel<DD, TQ_F32><<<g, 512, 0, s>>>(r);              \
-    else if (dtype == TQ_F16) dense_rotate_kernel<DD, TQ_F16><<<g, 512, 0, s>>>(r);         \
-    else dense_rotate_kernel<DD, TQ_BF16><<<g, 512, 0, s>>>(r);                             \
-  } break;
-    switch (DP) {
-      TQ_ROT_CASE(32)
-      TQ_ROT_CASE(64)
-      TQ_ROT_CASE(96)
-      TQ_ROT_CASE(128)
-      TQ_ROT_CASE(160)
-      TQ_ROT_CASE(192)
-      TQ_ROT_CASE(224)
-      TQ_ROT_CASE(256)
-    }
-#undef TQ_ROT_CASE
-  }
+  launch_rotate(q, dtype, B, Hq, Sq, d, sqb, sqh, sqs, key_pi_split, key_s_eff_f16, q_rot, seff_frag, cus, s);
   // P as f16 (hi, lo) where the term-by-term path keeps it so (its tiled kernel); one f16 where its
   // prefill kernel rounds it
   const bool plo = !prefill_applies(Hq, Hkv, d, bits, val_bits, mask != nullptr);
@@ -1264,8 +1386,8 @@ int tq_prefill_attention(const void* q, int32_t dtype, int64_t sqb, int64_t sqh,
   } else { TQ_DENSE_P(DD, NN, true) }
 #define TQ_DENSE_CASE(DD)                                                                      \
   case DD:                                                                                     \
-    if (dw) dense_expand_kernel<DD, true><<<egrid, 2 * DD, 0, s>>>(e);                         \
-    else dense_expand_kernel<DD, false><<<egrid, 2 * DD, 0, s>>>(e);                           \
+    if (dw) dense_expand_kernel<DD, true, true><<<egrid, 2 * DD, 0, s>>>(e);                   \
+    else dense_expand_kernel<DD, false, true><<<egrid, 2 * DD, 0, s>>>(e);                     \
     if (p.NW == 8) { if constexpr (dense_wide(DD)) { TQ_DENSE(DD, 8) } }                            \
     else { TQ_DENSE(DD, 4) }                                                                   \
     if (p.nsplit > 1) dense_merge_kernel<DD><<<mgrid, 2 * DD, 0, s>>>(a, p.NW);                \
@@ -1284,6 +1406,97 @@ int tq_prefill_attention(const void* q, int32_t dtype, int64_t sqb, int64_t sqh,
 #undef TQ_DENSE
 #undef TQ_DENSE_P
 #undef TQ_DENSE_R
+    const int st = launch_status(what);
+    if (st != TQ_OK) return st;
+  }
+  return TQ_OK;
+}
+
+int64_t tq_prefill_scores_workspace_size(int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Sk, int32_t d) {
+  if (!supported_dim(d) || B <= 0 || Hkv <= 0 || Hq <= 0 || Hq % Hkv || Sq <= 0 || Sk <= 0 || Sk >= (1 << 24)) return 0;
+  const int64_t groups = static_cast<int64_t>(B) * Hkv, group = score_group_bytes(Sk, d);
+  return dense_q_bytes(B, Hq, Sq, d) + std::min(groups, std::max<int64_t>(1, kDenseWorkspace / group)) * group;
+}
+
+int tq_prefill_scores(const void* q, int32_t dtype, int64_t sqb, int64_t sqh, int64_t sqs,
+                      const uint16_t* key_pi_split, const uint16_t* key_s_eff_f16, const uint8_t* key_codes,
+                      const uint8_t* key_signs, const uint16_t* key_rn, const uint16_t* key_vn,
+                      const uint16_t* key_centroids_f16, int32_t bits, int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq,
+                      int32_t Sk, int64_t kv_stride, int32_t d, float coeff, float* out, void* workspace,
+                      int64_t workspace_bytes, void* stream) {
+  const char* what = "tq_prefill_scores";
+  if (!supported_dim(d)) {
+    set_error("%s: head_dim %d not supported (multiples of 8 from 8 to 256)", what, (int)d);
+    return TQ_EUNSUPPORTED;
+  }
+  TQ_REQUIRE(bits >= 2 && bits <= 4, "%s: key bits must be in [2, 4], got %d", what, (int)bits);
+  TQ_REQUIRE(B >= 0 && Hq >= 0 && Hkv >= 1 && Sq >= 0 && Sk >= 0 && Hq % Hkv == 0, "%s: bad shape", what);
+  const int64_t ldk = kv_stride > 0 ? kv_stride : Sk;
+  TQ_REQUIRE(ldk >= Sk, "%s: kv_stride %lld < Sk %d", what, (long long)kv_stride, (int)Sk);
+  TQ_REQUIRE(dtype == TQ_F32 || dtype == TQ_F16 || dtype == TQ_BF16, "%s: unknown dtype %d", what, (int)dtype);
+  if (static_cast<int64_t>(B) * Hq * Sq * Sk == 0) return TQ_OK;
+  TQ_REQUIRE(Sk < (1 << 24), "%s: %d keys, fewer than 2^24 wanted", what, (int)Sk);
+  TQ_REQUIRE(q && key_pi_split && key_s_eff_f16 && key_codes && key_signs && key_rn && key_vn && key_centroids_f16 &&
+                 out && workspace,
+             "%s: null pointer", what);
+  TQ_REQUIRE(((reinterpret_cast<uintptr_t>(key_pi_split) | reinterpret_cast<uintptr_t>(workspace)) & 15) == 0,
+             "%s: key_pi_split and workspace must be 16-byte aligned", what);
+  const int cus = device_cus(), G = Hq / Hkv, DP = pad_dim(d);
+  const int64_t groups = static_cast<int64_t>(B) * Hkv, group = score_group_bytes(Sk, d);
+  const int64_t qbytes = dense_q_bytes(B, Hq, Sq, d);
+  const int64_t per = std::min(groups, (workspace_bytes - qbytes) / group);
+  TQ_REQUIRE(workspace_bytes >= qbytes && per >= 1, "%s: %lld workspace bytes, at least %lld needed", what,
+             (long long)workspace_bytes, (long long)(qbytes + group));
+  hipStream_t s = as_stream(stream);
+  uint16_t* seff_frag = static_cast<uint16_t*>(workspace);
+  uint16_t* q_rot = seff_frag + static_cast<int64_t>(DP) * DP;
+  launch_rotate(q, dtype, B, Hq, Sq, d, sqb, sqh, sqs, key_pi_split, key_s_eff_f16, q_rot, seff_frag, cus, s);
+  const bool dw = d % 32 == 0 && ((reinterpret_cast<uintptr_t>(key_codes) | reinterpret_cast<uintptr_t>(key_signs)) & 3) == 0;
+  const bool lines = Sk % 32 == 0 && reinterpret_cast<uintptr_t>(out) % 128 == 0;
+  uint8_t* tiles = static_cast<uint8_t*>(workspace) + qbytes;
+  DenseScoreArgs a{};
+  a.q_rot = q_rot; a.tiles = tiles;
+  a.Hq = Hq; a.Hkv = Hkv; a.Sq = Sq; a.Sk = Sk; a.d = d; a.G = G;
+  a.rchunks = (Sq + 31) / 32;
+  a.ntile = (Sk + kDenseKeys - 1) / kDenseKeys;
+  a.out = out;
+  TQ_REQUIRE(static_cast<int64_t>(G) * a.rchunks < (int64_t(1) << 31) && groups < (int64_t(1) << 31), "%s: too many rows",
+             what);
+  a.nblk = (G * a.rchunks + 3) / 4;
+  a.tfac = reinterpret_cast<float*>(tiles + per * a.ntile * static_cast<int64_t>(2 * DP * 64));
+  // about eight blocks per compute unit, of at least four tiles
+  const int64_t blocks = std::min(per, groups) * a.nblk;
+  a.cpt = static_cast<int>(std::min<int64_t>(a.ntile, std::max<int64_t>(4, blocks * a.ntile / (8LL * cus))));
+  const int nsplit = (a.ntile + a.cpt - 1) / a.cpt;
+  TQ_REQUIRE(blocks * nsplit < (int64_t(1) << 31), "%s: too many blocks", what);
+  for (int64_t g0 = 0; g0 < groups; g0 += per) {
+    a.nbh = static_cast<int>(std::min(per, groups - g0));
+    a.bh0 = g0;
+    ExpandArgs e{};
+    e.kcodes = key_codes; e.ksigns = key_signs; e.krn = key_rn; e.kvn = key_vn; e.kcent = key_centroids_f16;
+    e.seff_frag = seff_frag; e.Sk = Sk; e.d = d; e.kb = bits - 1; e.vb = 1; e.ntile = a.ntile;
+    e.ldk = ldk; e.bh0 = g0; e.total = static_cast<int64_t>(a.nbh) * a.ntile;
+    e.coeff = coeff; e.tiles = tiles; e.tfac = const_cast<float*>(a.tfac);
+    const unsigned egrid = static_cast<unsigned>(std::min<int64_t>(e.total, 8LL * cus));
+    const unsigned grid = static_cast<unsigned>(a.nbh) * a.nblk * nsplit;
+#define TQ_SCORES_CASE(DD)                                                                     \
+  case DD:                                                                                     \
+    if (dw) dense_expand_kernel<DD, true, false><<<egrid, 2 * DD, 0, s>>>(e);                  \
+    else dense_expand_kernel<DD, false, false><<<egrid, 2 * DD, 0, s>>>(e);                    \
+    if (lines) dense_scores_kernel<DD, true><<<grid, 256, 0, s>>>(a);                          \
+    else dense_scores_kernel<DD, false><<<grid, 256, 0, s>>>(a);                               \
+    break;
+    switch (DP) {
+      TQ_SCORES_CASE(32)
+      TQ_SCORES_CASE(64)
+      TQ_SCORES_CASE(96)
+      TQ_SCORES_CASE(128)
+      TQ_SCORES_CASE(160)
+      TQ_SCORES_CASE(192)
+      TQ_SCORES_CASE(224)
+      TQ_SCORES_CASE(256)
+    }
+#undef TQ_SCORES_CASE
     const int st = launch_status(what);
     if (st != TQ_OK) return st;
   }

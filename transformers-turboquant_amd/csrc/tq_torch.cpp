@@ -649,6 +649,53 @@ Tensor attend(const Tensor& q_in, const Tensor& pi_split, const Tensor& s_eff16,
   return out;
 }
 
+// Materialised scores of raw queries: tq_prefill_scores past the 128 columns (query rows x group) per
+// kv head that one block of the packed-plane kernels holds (32/8 heads: 33 rows x 4096 keys 371 us
+// packed, 39 expanded; up to 128 columns those split the keys and read them once), otherwise query_prep
+// and scores.
+bool score_route(int64_t B, int64_t Hq, int64_t hkv, int64_t Sq, int64_t sk, int64_t D, int64_t bits) {
+  if (B < 1 || Hq < 1 || Sq < 1 || sk < 1 || sk >= (int64_t{1} << 24) || bits < 2 || bits > 4) return false;
+  if (D < 8 || D > 256 || D % 8 != 0) return false;
+  return Hq / hkv * Sq > 128;
+}
+
+Tensor attend_scores_meta(const Tensor& q, const Tensor& pi_split, const Tensor& s_eff16, const Tensor& codes,
+                          const Tensor& signs, const Tensor& rn, const Tensor& vn, const Tensor& cent16, int64_t bits,
+                          int64_t hkv, int64_t sk, int64_t kv_stride, double coeff) {
+  const Checker c{"tq::attend_scores", q.device()};
+  TORCH_CHECK(q.dim() == 4, c.op, ": expected [B, Hq, Sq, D] queries");
+  const int64_t D = q.size(3);
+  c.table(pi_split, "split Pi", at::kHalf, 2 * D * D);
+  c.table(s_eff16, "f16 S_eff", at::kHalf, D * D);
+  check_keys(c, q, codes, signs, rn, vn, cent16, bits, hkv, sk, kv_stride);
+  return at::empty({q.size(0), q.size(1), q.size(2), sk}, q.options().dtype(at::kFloat));
+}
+
+Tensor attend_scores(const Tensor& q_in, const Tensor& pi_split, const Tensor& s_eff16, const Tensor& codes,
+                     const Tensor& signs, const Tensor& rn, const Tensor& vn, const Tensor& cent16, int64_t bits,
+                     int64_t hkv, int64_t sk, int64_t kv_stride, double coeff) {
+  if (!(q_in.dim() == 4 && hkv >= 1 && q_in.size(1) % hkv == 0 &&
+        score_route(q_in.size(0), q_in.size(1), hkv, q_in.size(2), sk, q_in.size(3), bits))) {
+    auto qp = query_prep(q_in, pi_split, s_eff16);
+    return scores(std::get<0>(qp), std::get<1>(qp), codes, signs, rn, vn, cent16, bits, hkv, sk, kv_stride, coeff);
+  }
+  Tensor out = attend_scores_meta(q_in, pi_split, s_eff16, codes, signs, rn, vn, cent16, bits, hkv, sk, kv_stride, coeff);
+  const c10::DeviceGuard g(q_in.device());
+  Tensor q = activation(q_in);
+  const int32_t B = static_cast<int32_t>(q.size(0)), Hq = static_cast<int32_t>(q.size(1)),
+                Sq = static_cast<int32_t>(q.size(2)), D = static_cast<int32_t>(q.size(3)),
+                Hkv = static_cast<int32_t>(hkv), Sk = static_cast<int32_t>(sk);
+  const int64_t bytes = tq_prefill_scores_workspace_size(B, Hq, Hkv, Sq, Sk, D);
+  Tensor ws = at::empty({bytes}, q.options().dtype(at::kByte));
+  check_status(tq_prefill_scores(q.data_ptr(), dtype_code(q.scalar_type()), q.stride(0), q.stride(1), q.stride(2),
+                                 ptr<uint16_t>(pi_split), ptr<uint16_t>(s_eff16), ptr<uint8_t>(codes),
+                                 ptr<uint8_t>(signs), ptr<uint16_t>(rn), ptr<uint16_t>(vn), ptr<uint16_t>(cent16),
+                                 static_cast<int32_t>(bits), B, Hq, Hkv, Sq, Sk, kv_stride, D,
+                                 static_cast<float>(coeff), ptr<float>(out), ws.data_ptr(), bytes, stream_of(out)),
+               "asymmetric_attention_scores");
+  return out;
+}
+
 // A cached decode step in one call: cache_append (the new keys / values into the capacity
 // planes at row pos, the new queries prepared in the same launch), then attention over the
 // planes' first pos + S rows.  The same two operators back to back, without the second
@@ -728,6 +775,8 @@ TORCH_LIBRARY(tq, m) {
         "Tensor kcent, int bits, Tensor vcodes, Tensor vvn, Tensor vcent, int val_bits, Tensor vpit, int hkv, "
         "int sk, int kv_stride, float coeff, float scale, bool causal, Tensor? mask, ScalarType out_dtype, "
         "int workspace) -> Tensor");
+  m.def("attend_scores(Tensor q, Tensor pi_split, Tensor s_eff, Tensor codes, Tensor signs, Tensor rn, Tensor vn, "
+        "Tensor centroids, int bits, int hkv, int sk, int kv_stride, float coeff) -> Tensor");
   m.def("cache_attend(Tensor k, Tensor v, Tensor q, Tensor kpi, Tensor kseff, Tensor kcent, Tensor kbounds, "
         "int key_code_bits, Tensor vpi, Tensor vbounds, int val_bits, Tensor kseff16, Tensor(a!) kcodes, "
         "Tensor(b!) ksigns, Tensor(c!) krn, Tensor(d!) kvn, Tensor(e!) vcodes, Tensor(f!) vvn, int pos, "
@@ -749,6 +798,7 @@ TORCH_LIBRARY_IMPL(tq, CUDA, m) {
   m.impl("scores", &scores);
   m.impl("attention", &attention);
   m.impl("attend", &attend);
+  m.impl("attend_scores", &attend_scores);
   m.impl("cache_attend", &cache_attend);
 }
 
@@ -766,5 +816,6 @@ TORCH_LIBRARY_IMPL(tq, Meta, m) {
   m.impl("scores", &scores_meta);
   m.impl("attention", &attention_meta);
   m.impl("attend", &attend_meta);
+  m.impl("attend_scores", &attend_scores_meta);
   m.impl("cache_attend", &cache_attend_meta);
 }

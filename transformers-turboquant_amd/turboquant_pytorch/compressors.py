@@ -21,7 +21,6 @@ import torch
 
 from ._ops import ops
 from .codebook import codebook, gaussian_matrix, midpoints, random_rotation, split_f16
-from .kernels.attention import scores_from_prepared
 
 __all__ = ["TurboQuantCompressorV2", "TurboQuantCompressorMSE"]
 
@@ -148,13 +147,12 @@ class TurboQuantCompressorV2:
                 raise ValueError("packed key planes live on the GPU; pass GPU queries")
             if Hq % Hk:
                 raise ValueError(f"query heads {Hq} not a multiple of compressed heads {Hk}")
-            q_rot, q_proj = self.prepare_queries(queries)
             t = _tables(self, queries.device, with_qjl=True)
             coeff = math.sqrt(math.pi / 2) / self.S.shape[0]
-            return scores_from_prepared(
-                q_rot, q_proj, compressed["packed_key_indices"], compressed["packed_qjl_signs"],
-                compressed["residual_norm"], compressed["vec_norms"], t.cent16, self.mse_bits + 1,
-                coeff, Hk, Sk, int(compressed.get("kv_stride", Sk)))
+            return ops().attend_scores(
+                queries, t.pi_split, t.s_eff16, compressed["packed_key_indices"], compressed["packed_qjl_signs"],
+                compressed["residual_norm"], compressed["vec_norms"], t.cent16, self.mse_bits + 1, Hk, int(Sk),
+                int(compressed.get("kv_stride", Sk)), float(coeff))
         # reference PyTorch branch (compressors.py:201-224)
         k_mse = compressed["k_mse"].float()
         signs = compressed["qjl_signs"].float()
