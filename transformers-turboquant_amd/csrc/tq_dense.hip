@@ -20,11 +20,11 @@
 // neither hi nor lo leaves f16's normal range at any key norm.
 //
 // Bound and measurements (bits 3, 32 / 8 heads, head_dim 128, against tq_query_prep and the
-// term-by-term prefill kernel, one MI355X): 8192 causal rows 1190 -> 880 us for the whole layer,
-// the attention kernel 1110 -> 765 us, 1.1 PFLOP/s on the matrix cores where a large library
+// term-by-term prefill kernel, one MI355X): 8192 causal rows 1160 -> 815 us for the whole layer,
+// the attention kernel 1110 -> 730 us, 1.15 PFLOP/s on the matrix cores where a large library
 // product reaches 1.3 (both hold the clock below 2 GHz); 512 rows over 16k cached keys 731 -> 245
 // us (blocks split the keys, the term-by-term kernel ran 128 blocks); head_dim 80, 1531 rows, 32
-// heads: 247 -> 105 us without the compressions.  A tile takes a compute unit 0.94 us with two
+// heads: 247 -> 95 us without the compressions.  A tile takes a compute unit 0.90 us with two
 // waves per SIMD (its matrix work alone 0.64 at 2.4 GHz); the rest is the chain scores -> softmax ->
 // P.V and the barrier.  Expansion is bound by its 6 bytes written per element (8 us per 16 MB).
 #include "tq_common.h"
@@ -422,7 +422,11 @@ struct DenseCfg {
   static constexpr int FIT = (KIB * 1024 - MB) / REC;
   static constexpr int NS = FIT >= 6 ? 6 : FIT;
   static constexpr int WPE = NW == 8 ? 2 : RES;  // waves per SIMD
-  static_assert(NS >= 3 && (NS - 3) * CPW < 64, "ring");
+  // six slots allow one block barrier per two tiles, with copies NS - 2 tiles ahead instead of NS - 1
+  // (a tile of 256 columns at head_dim 128: 0.94 -> 0.90 us; of 128 at head_dim 64: 0.45 -> 0.43)
+  static constexpr bool PAIR = NS == 6 && !MASK;
+  static constexpr int LEAD = PAIR ? NS - 2 : NS - 1;
+  static_assert(NS >= 3 && (LEAD - 2) * CPW < 64, "ring");
 };
 
 // Block -> work: query blocks heavy first across every (batch, kv head); consecutive blocks are
@@ -573,7 +577,7 @@ __attribute__((amdgpu_waves_per_eu(DenseCfg<DP, NW, MASK, RES>::WPE)))
 dense_attn_kernel(DenseArgs a) {
   using C = DenseCfg<DP, NW, MASK, RES>;
   constexpr bool MDMA = C::MDMA;
-  constexpr int KS = C::KS, DB = C::DB, REC = C::REC, NS = C::NS, CPW = C::CPW, NF = REC / 1024;
+  constexpr int KS = C::KS, DB = C::DB, REC = C::REC, NS = C::NS, CPW = C::CPW, NF = REC / 1024, LEAD = C::LEAD;
   constexpr float LOG2E = 1.4426950408889634f;
   constexpr float TAU = 8.0f;  // lazy-rescale headroom (log2 units)
   __shared__ __attribute__((aligned(16))) uint8_t ring[NS * REC];
@@ -606,8 +610,10 @@ dense_attn_kernel(DenseArgs a) {
       qf[ks] = real ? v : half8{};
     }
   }
-  // this wave's tiles end at tw (its last row's last key); tiles from tf on need masking
+  // this wave's tiles end at tw (its last row's last key); tiles from tf on need masking, tiles before
+  // tfb in no wave of the block.  A wave without columns (tw = tb) only copies
   int tw = te, tf = te;
+  const int tfb = min(te, (a.causal ? min(qblk * a.QT + off + 1, a.Sk) : a.Sk) / kDenseKeys);
   {
     const int ql0 = wave * 32 / a.G, ql1 = min((wave * 32 + 31) / a.G, a.QT - 1);
     const int i0 = qblk * a.QT + ql0, i1 = min(qblk * a.QT + ql1, a.Sq - 1);
@@ -665,11 +671,11 @@ dense_attn_kernel(DenseArgs a) {
     if (--left > 0) src += REC;
     dst = dst + REC == ring_lds + NS * REC ? ring_lds : dst + REC;
   };
-  // the record issued NS - 3 calls before the latest one has landed (this wave's copies)
+  // the record issued LEAD - 2 calls before the latest one has landed (this wave's copies)
   auto landed = [&]() __attribute__((always_inline)) {
     // mask copies of a tile are issued one iteration ahead, before that iteration's record
     if constexpr (MASK) wait_vm<(NS > 3 ? CPW : 0)>();
-    else wait_vm<(NS - 3) * CPW>();
+    else wait_vm<(LEAD - 2) * CPW>();
   };
   auto block_sync = [&]() __attribute__((always_inline)) {
     wait_lds();  // this wave's fragment reads are done: their slot may be overwritten
@@ -867,13 +873,13 @@ dense_attn_kernel(DenseArgs a) {
   factors(tb);  // and waits for q: the ring's waits count copies only
   if (te > tb) {
 #pragma unroll
-    for (int i = 0; i < NS - 1; ++i) {
+    for (int i = 0; i < LEAD; ++i) {
       issue();
       if (i == 0) {
         if constexpr (MASK) issue_mask(tb);
       }
     }
-    wait_vm<MASK ? 0 : (NS - 2) * CPW>();
+    wait_vm<MASK ? 0 : (LEAD - 1) * CPW>();
     if constexpr (MASK) {
       issue_mask(tb + 1);
       if (NS > 3) wait_vm<0>();  // the first advance() leaves CPW copies in flight, not these
@@ -884,7 +890,7 @@ dense_attn_kernel(DenseArgs a) {
     const uint8_t* cur = ring0;  // tile t's record
     if (tb < tw) first_scores(tb, cur);
     auto next = [&](const uint8_t* p) { return p + REC == ring1 ? ring0 : p + REC; };
-    // tile t + 1 landed for every wave, every wave done with tile t - 1, whose slot takes tile t + NS - 1
+    // tile t + 1 landed for every wave, every wave done with tile t - 1: the slot of tile t + LEAD is free
     auto advance = [&](int t) __attribute__((always_inline)) {
       if (((t + 1 - tb) & 63) == 0) factors(t + 1);
       landed();
@@ -893,6 +899,29 @@ dense_attn_kernel(DenseArgs a) {
       issue();
     };
     int t = tb;
+    if constexpr (C::PAIR) {
+      // two tiles per barrier while the block's tiles need no masking (tfb: the same for its waves):
+      // tiles t + 1 and t + 2 have landed, every wave is done with t - 1, so the slots of t - 2 and t - 1
+      // take t + 4 and t + 5
+      for (; t + 2 < tfb; t += 2) {
+        if (((t + 1 - tb) & 63) == 0) factors(t + 1);
+        wait_vm<(LEAD - 3) * CPW>();
+        block_sync();
+        issue();
+        issue();
+        const uint8_t* nxt = next(cur);
+        if (tb < tw) {
+          tile(t, cur, nxt, std::true_type{});
+          settle(max16());
+        }
+        if (((t + 2 - tb) & 63) == 0) factors(t + 2);
+        cur = next(nxt);
+        if (tb < tw) {
+          tile(t + 1, nxt, cur, std::true_type{});
+          settle(max16());
+        }
+      }
+    }
     for (; t + 1 < tf; ++t) {  // the next tile needs no masking
       advance(t);
       const uint8_t* nxt = next(cur);
@@ -1158,7 +1187,8 @@ static int device_cus() {
 }
 
 // Block size and key splits for the smallest estimated time.  Unit: the time a compute unit takes for
-// one tile of 256 columns (two waves per SIMD; a lone 4-wave block takes kLone of it).  A block adds
+// one tile of 256 columns (two waves per SIMD; a lone 4-wave block takes kLone of it, two of them
+// kNarrow, kUnfilled where they leave some units to one).  A block adds
 // kBlock (query fragments, first copies, output rotation), a split its partial sums through memory
 // and the merge launch.
 // Blocks that fit a compute unit together (LDS, and 256 VGPRs a wave up to head_dim 160)
@@ -1168,7 +1198,7 @@ constexpr int dense_resident(int DP, int NW, bool masked) {
 }
 // Head dims with an 8-wave form
 constexpr bool dense_wide(int DP) { return DP == 96 || DP == 128; }
-constexpr double kLone = 0.7, kBlock = 4.0, kMergeLaunch = 4.0, kPart = 0.04, kNarrow = 1.02;
+constexpr double kLone = 0.7, kBlock = 4.0, kMergeLaunch = 4.0, kPart = 0.04, kNarrow = 1.02, kUnfilled = 0.95;
 
 static DensePlan dense_plan(int64_t groups, int G, int Sq, int Sk, int d, bool causal, bool masked, int cus) {
   const int DP = pad_dim(d);
@@ -1204,7 +1234,7 @@ static DensePlan dense_plan(int64_t groups, int G, int Sq, int Sk, int d, bool c
       const double work = mean * scale, blocks = pieces * scale;
       const double per_cu = std::min<double>(resident, std::ceil(blocks / cus));
       // time of one tile of one block: `per_cu` blocks of NW waves share the compute unit
-      const double tile = NW == 8 ? 1.0 : per_cu > 1 ? 0.5 * kNarrow * per_cu : kLone;
+      const double tile = NW == 8 ? 1.0 : per_cu > 1 ? 0.5 * per_cu * (blocks < cus * per_cu ? kUnfilled : kNarrow) : kLone;
       const double slots = cus * per_cu;
       const double even = (work + kBlock * blocks) / slots * tile;
       const double rounds = std::ceil(blocks / slots - 0.02);
