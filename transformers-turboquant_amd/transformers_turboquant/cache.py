@@ -154,8 +154,9 @@ class TurboQuantCacheLayer(CacheLayerMixin):
                       out_dtype: torch.dtype = torch.float32) -> torch.Tensor:
         """GPU: append_prepare() followed by attention over every cached position
         (turboquant_pytorch.fused.attention_from_prepared), in one operator call
-        (tq::cache_attend): the same kernels and results, without the second operator's host
-        cost, which bounds a one-token decode step.  Returns the attention output [B, S_q, Hq, D]."""
+        (tq::cache_attend), without the second operator's host cost, which bounds a one-token
+        decode step.  A prompt chunk of many rows attends over keys expanded once
+        (tq_prefill_attention) instead of the packed planes.  Returns [B, S_q, Hq, D]."""
         if k.device.type != "cuda":
             raise ValueError("append_attend runs on the GPU; use append_prepare on the CPU")
         B, H, S, D = k.shape

@@ -13,9 +13,9 @@ value planes once per block of query rows, runs an online softmax in f32, and
 accumulates P.V in the value compressor's rotated domain, applying Pi_v once
 per output row.  Grouped-query attention is served without expanding K/V.
 Many query rows (prompts, prompt chunks) score against keys expanded once per call
-(tq_prefill_attention; its workspace comes from torch).  Few-query (decode) shapes take a split-K path whose partial results live in a
-workspace that the op allocates from torch (tq_attention_workspace_size bytes), or
-in the library's own scratch array (split_k="static").
+(tq_prefill_attention; its workspace comes from torch).  Few-query (decode) shapes take a
+split-K path whose partial results live in a workspace that the op allocates from torch
+(tq_attention_workspace_size bytes), or in the library's own scratch array (split_k="static").
 
 A compressed dict may carry ``kv_stride``: its planes then hold ``kv_stride``
 positions per (batch, kv head) of which the first ``shape[2]`` are attended
