@@ -82,6 +82,7 @@ def _err(got, ref):
     (64, 2, 1, 4, 2, 70, 31, False),       # fewer keys than a tile
     (32, 3, 3, 8, 2, 100, 257, False),
     (40, 2, 2, 4, 4, 130, 600, True),      # 5-byte sign rows: byte loads
+    (48, 3, 4, 8, 2, 100, 900, True),      # 6-byte sign rows: 16-bit loads
     (80, 3, 3, 8, 2, 65, 530, True),
     (96, 4, 3, 6, 2, 90, 200, True),
     (112, 3, 3, 4, 1, 50, 90, False),

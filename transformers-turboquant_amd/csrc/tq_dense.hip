@@ -235,13 +235,15 @@ struct Field32 {
     return __builtin_amdgcn_alignbit(hi, lo, bit & 31);
   }
 };
-// DW: rows are whole dwords (head_dim a multiple of 32); otherwise byte loads of the real bytes
-template <bool DW>
+// W: bytes per load.  Rows are whole dwords at head dims that are multiples of 32, whole 16-bit
+// words at other multiples of 16 (head_dim 80, 32 x 1531 keys: the expansion takes 18.3 us, by single
+// bytes 21.4), single bytes otherwise
+template <int W>
 __device__ __forceinline__ Field32 load_field(const uint8_t* row, int blk, int b, int d) {
   Field32 f;
 #pragma unroll
   for (int i = 0; i < 4; ++i) f.w[i] = 0;
-  if constexpr (DW) {
+  if constexpr (W == 4) {
     const uint32_t* p = reinterpret_cast<const uint32_t*>(row) + blk * b;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -250,8 +252,11 @@ __device__ __forceinline__ Field32 load_field(const uint8_t* row, int blk, int b
     const int n = min(32, d - 32 * blk) * b / 8;  // real bytes of the field
     const uint8_t* p = row + 4 * blk * b;
 #pragma unroll
-    for (int i = 0; i < 16; ++i)
-      if (i < n) f.w[i >> 2] |= static_cast<uint32_t>(p[i]) << (8 * (i & 3));
+    for (int i = 0; i < 16 / W; ++i)
+      if (W * i < n) {
+        const uint32_t v = W == 2 ? reinterpret_cast<const uint16_t*>(p)[i] : p[i];
+        f.w[W * i >> 2] |= v << (8 * (W * i & 3));
+      }
   }
   return f;
 }
@@ -259,7 +264,7 @@ __device__ __forceinline__ Field32 load_field(const uint8_t* row, int blk, int b
 // One wave per 32-dim block; blocks walk the tiles.  Lane (key n, half h) of wave w ends with
 // dims 32w + 16s + 8h + 0..7 (s = 0, 1) of its key: exactly its 16 bytes of k^ fragments 2w + s.
 // V^ is transposed through a wave-private LDS tile.
-template <int DP, bool DW, bool VALS>
+template <int DP, int W, bool VALS>
 __global__ void __launch_bounds__(2 * DP) dense_expand_kernel(ExpandArgs a) {
   constexpr int KS = DP / 16, NW = DP / 32;
   constexpr int VP = 36;  // halves per row of the V^ transposition tile
@@ -305,9 +310,9 @@ __global__ void __launch_bounds__(2 * DP) dense_expand_kernel(ExpandArgs a) {
     Raw r;
     r.ok = k0 + n < a.Sk;
 #pragma unroll
-    for (int i = 0; i < NW; ++i) r.sw[i] = load_field<DW>(a.ksigns + row * sc, i, 1, d).w[0];
-    r.kf = load_field<DW>(a.kcodes + row * kc, w, a.kb, d);
-    if constexpr (VALS) r.vf = load_field<DW>(a.vcodes + row * vc, w, a.vb, d);
+    for (int i = 0; i < NW; ++i) r.sw[i] = load_field<W>(a.ksigns + row * sc, i, 1, d).w[0];
+    r.kf = load_field<W>(a.kcodes + row * kc, w, a.kb, d);
+    if constexpr (VALS) r.vf = load_field<W>(a.vcodes + row * vc, w, a.vb, d);
     r.vn = a.kvn[row];
     r.rn = a.krn[row];
     if constexpr (VALS) r.vvn = a.vvn[row];
@@ -1280,6 +1285,11 @@ static int64_t score_group_bytes(int Sk, int d) {
   return nt * (2 * pad_dim(d) * 64) + (nt * 4 + 15) / 16 * 16;
 }
 
+// Bytes per load that every packed row (d / 8 bytes per code bit) and plane base allows the expansion
+static int row_width(int d, uintptr_t bases) {
+  return d % 32 == 0 && bases % 4 == 0 ? 4 : d % 16 == 0 && bases % 2 == 0 ? 2 : 1;
+}
+
 // q_rot, and S_eff's fragments for the expansion
 static void launch_rotate(const void* q, int dtype, int B, int Hq, int Sq, int d, int64_t sqb, int64_t sqh, int64_t sqs,
                           const uint16_t* key_pi_split, const uint16_t* key_s_eff_f16, uint16_t* q_rot,
@@ -1379,9 +1389,8 @@ int tq_prefill_attention(const void* q, int32_t dtype, int64_t sqb, int64_t sqh,
   // P as f16 (hi, lo) where the term-by-term path keeps it so (its tiled kernel); one f16 where its
   // prefill kernel rounds it
   const bool plo = !prefill_applies(Hq, Hkv, d, bits, val_bits, mask != nullptr);
-  // rows of whole dwords
-  const bool dw = d % 32 == 0 && ((reinterpret_cast<uintptr_t>(key_codes) | reinterpret_cast<uintptr_t>(key_signs) |
-                                   reinterpret_cast<uintptr_t>(val_codes)) & 3) == 0;
+  const int width = row_width(d, reinterpret_cast<uintptr_t>(key_codes) | reinterpret_cast<uintptr_t>(key_signs) |
+                                     reinterpret_cast<uintptr_t>(val_codes));
   uint8_t* tiles = static_cast<uint8_t*>(workspace) + qbytes;
   float* part_o = reinterpret_cast<float*>(tiles + per * p.ntile * (3 * DP * 64));
   float* part_ml = part_o + (p.nsplit > 1 ? per * recs * DP * 32 : 0);
@@ -1416,8 +1425,9 @@ int tq_prefill_attention(const void* q, int32_t dtype, int64_t sqb, int64_t sqh,
   } else { TQ_DENSE_P(DD, NN, true) }
 #define TQ_DENSE_CASE(DD)                                                                      \
   case DD:                                                                                     \
-    if (dw) dense_expand_kernel<DD, true, true><<<egrid, 2 * DD, 0, s>>>(e);                   \
-    else dense_expand_kernel<DD, false, true><<<egrid, 2 * DD, 0, s>>>(e);                     \
+    if (width == 4) dense_expand_kernel<DD, 4, true><<<egrid, 2 * DD, 0, s>>>(e);              \
+    else if (width == 2) dense_expand_kernel<DD, 2, true><<<egrid, 2 * DD, 0, s>>>(e);         \
+    else dense_expand_kernel<DD, 1, true><<<egrid, 2 * DD, 0, s>>>(e);                         \
     if (p.NW == 8) { if constexpr (dense_wide(DD)) { TQ_DENSE(DD, 8) } }                            \
     else { TQ_DENSE(DD, 4) }                                                                   \
     if (p.nsplit > 1) dense_merge_kernel<DD><<<mgrid, 2 * DD, 0, s>>>(a, p.NW);                \
@@ -1481,7 +1491,7 @@ int tq_prefill_scores(const void* q, int32_t dtype, int64_t sqb, int64_t sqh, in
   uint16_t* seff_frag = static_cast<uint16_t*>(workspace);
   uint16_t* q_rot = seff_frag + static_cast<int64_t>(DP) * DP;
   launch_rotate(q, dtype, B, Hq, Sq, d, sqb, sqh, sqs, key_pi_split, key_s_eff_f16, q_rot, seff_frag, cus, s);
-  const bool dw = d % 32 == 0 && ((reinterpret_cast<uintptr_t>(key_codes) | reinterpret_cast<uintptr_t>(key_signs)) & 3) == 0;
+  const int width = row_width(d, reinterpret_cast<uintptr_t>(key_codes) | reinterpret_cast<uintptr_t>(key_signs));
   const bool lines = Sk % 32 == 0 && reinterpret_cast<uintptr_t>(out) % 128 == 0;
   uint8_t* tiles = static_cast<uint8_t*>(workspace) + qbytes;
   DenseScoreArgs a{};
@@ -1511,8 +1521,9 @@ int tq_prefill_scores(const void* q, int32_t dtype, int64_t sqb, int64_t sqh, in
     const unsigned grid = static_cast<unsigned>(a.nbh) * a.nblk * nsplit;
 #define TQ_SCORES_CASE(DD)                                                                     \
   case DD:                                                                                     \
-    if (dw) dense_expand_kernel<DD, true, false><<<egrid, 2 * DD, 0, s>>>(e);                  \
-    else dense_expand_kernel<DD, false, false><<<egrid, 2 * DD, 0, s>>>(e);                    \
+    if (width == 4) dense_expand_kernel<DD, 4, false><<<egrid, 2 * DD, 0, s>>>(e);             \
+    else if (width == 2) dense_expand_kernel<DD, 2, false><<<egrid, 2 * DD, 0, s>>>(e);        \
+    else dense_expand_kernel<DD, 1, false><<<egrid, 2 * DD, 0, s>>>(e);                        \
     if (lines) dense_scores_kernel<DD, true><<<grid, 256, 0, s>>>(a);                          \
     else dense_scores_kernel<DD, false><<<grid, 256, 0, s>>>(a);                               \
     break;
