@@ -70,6 +70,31 @@ def _err(got, ref):
     return ((got.double() - ref).norm() / ref.norm()).item()
 
 
+_DT = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
+
+
+def _direct(q, kc, vc, ck, cv, mask=None, causal=False, out_dtype=torch.float32):
+    """tq_prefill_attention through the C ABI: no choice of route, the mask as it lies in memory."""
+    B, hq, sq, d = q.shape
+    _, hkv, sk, _ = ck["shape"]
+    tk, tv = _tables(kc, q.device, True), _tables(vc, q.device, False)
+    lib, p = _native.lib(), _native.ptr
+    m = mask.expand(B, hq, sq, sk) if mask is not None else None
+    nb = lib.tq_prefill_workspace_size(B, hq, hkv, sq, sk, d, int(causal), int(m is not None))
+    ws = torch.empty(nb, dtype=torch.uint8, device=DEV)
+    out = torch.zeros(B, sq, hq, d, device=DEV, dtype=out_dtype)
+    st = lib.tq_prefill_attention(
+        p(q), _DT[q.dtype], q.stride(0), q.stride(1), q.stride(2), p(tk.pi_split), p(tk.s_eff16),
+        p(ck["packed_key_indices"]), p(ck["packed_qjl_signs"]), p(ck["residual_norm"]), p(ck["vec_norms"]),
+        p(tk.cent16), kc.mse_bits + 1, p(cv["packed_indices"]), p(cv["vec_norms"]), p(tv.cent32), vc.bits,
+        p(tv.pit_split), B, hq, hkv, sq, sk, 0, d, math.sqrt(math.pi / 2) / d, 1 / math.sqrt(d), int(causal),
+        p(m) if m is not None else None, _DT[m.dtype] if m is not None else 0,
+        *(m.stride() if m is not None else (0, 0, 0, 0)), p(out), _DT[out_dtype], p(ws), ctypes.c_int64(nb),
+        torch.cuda.current_stream().cuda_stream)
+    assert st == 0, lib.tq_last_error()
+    return out
+
+
 @pytest.mark.parametrize("d,bits,vbits,hq,hkv,sq,sk,causal", [
     (128, 3, 3, 8, 2, 64, 64, True),       # one block of 256 columns, whole tiles
     (128, 2, 2, 8, 2, 65, 65, True),       # a second block and a second tile of one row / key
@@ -116,6 +141,30 @@ def test_prefill_masks(d, mdt, sk, layout):
         m = m.transpose(-1, -2).contiguous().transpose(-1, -2)
     got = compressed_attention(q, kc, vc, ck, cv, attention_mask=m)
     assert _err(got, _reference(q, kc, vc, ck, cv, mask=m.expand(B, hq, sq, sk))) < REL
+
+
+@pytest.mark.parametrize("d", [64, 80, 128])
+@pytest.mark.parametrize("mdt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows", ["query", "padding"])
+def test_prefill_masks_sliced_to_an_odd_key_count(d, mdt, rows):
+    """16-bit masks cut from a wider buffer: every row starts on a dword and ends inside one.  The last
+    key, masked in half of the rows, counts as any other, and the buffer's values past it (they would
+    raise a key's weight to 1) are never used.  1101 keys: the operator takes the expanded kernels at
+    every head dim; the C entry takes the mask where it lies."""
+    print("case:", d, mdt, rows, flush=True)
+    sq, sk, hq, hkv, B = 100, 1101, 8, 2, 2
+    kc, vc, q, ck, cv = _make(d, 3, 3, hq, hkv, sq, sk)
+    g = torch.Generator(device=DEV).manual_seed(sk)
+    n = sq if rows == "query" else 1
+    wide = torch.full((B, 1, n, 1200), 60.0, device=DEV, dtype=mdt)
+    m = wide[..., :sk]
+    m.copy_(torch.randn(B, 1, n, sk, device=DEV, generator=g))
+    m[..., sk - 1] = 30.0                       # the last key outweighs every other one ...
+    m[0, ..., sk - 1] = torch.finfo(mdt).min    # ... or has no weight
+    m[1, :, : n // 2, sk - 1] = torch.finfo(mdt).min
+    ref = _reference(q, kc, vc, ck, cv, mask=m.expand(B, hq, sq, sk))
+    assert _err(compressed_attention(q, kc, vc, ck, cv, attention_mask=m), ref) < REL
+    assert _err(_direct(q, kc, vc, ck, cv, mask=m), ref) < REL
 
 
 def test_prefill_rows_without_a_real_key():

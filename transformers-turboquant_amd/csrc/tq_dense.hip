@@ -629,7 +629,9 @@ dense_attn_kernel(DenseArgs a) {
   }
   // The mask reaches a lane through LDS: a tile's 32 columns x 32 keys as whole row segments
   // (64 or 128 bytes per column, copied one tile ahead) instead of 8- or 16-byte pieces of 32 rows
-  // per load.  Rows must start on dwords and be contiguous in keys; others are read directly.
+  // per load.  Rows must be whole dwords from a dword on and contiguous in keys (a 16-bit row of an odd
+  // key count ends inside a dword: its copy would read past the mask or drop the last key); others are
+  // read directly.
   // Segment c of column r sits at chunk c ^ (r's bits that pick its banks): conflict-free reads.
   [[maybe_unused]] const uint8_t* mrow = nullptr;
   [[maybe_unused]] const uint8_t* mbase = nullptr;
@@ -646,7 +648,7 @@ dense_attn_kernel(DenseArgs a) {
     mrow = mbase + at(c) * es;
     const int64_t far = (a.G - 1) * (a.smh < 0 ? -a.smh : a.smh) + a.QT * (a.smq < 0 ? -a.smq : a.smq) + a.Sk;
     mdma = MDMA && a.smk == 1 && a.smh >= 0 && a.smq >= 0 && far * es < (int64_t(1) << 31) &&
-           (reinterpret_cast<uintptr_t>(a.mask) & 3) == 0 && ((a.smb | a.smh | a.smq) * es & 3) == 0;
+           (reinterpret_cast<uintptr_t>(a.mask) & 3) == 0 && ((a.smb | a.smh | a.smq | a.Sk) * es & 3) == 0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int r = m32 ? 8 * i + (lane >> 3) : 16 * (i & 1) + (lane >> 2);

@@ -152,8 +152,9 @@ void check_values(const Checker& c, const Tensor& q_rot, const Tensor& vcodes, c
 // the additive mask as a float32 view broadcast to [B, Hq, Sq, Sk] (no copy when it already
 // is float32 on the device); `own_type`: float16 and bfloat16 masks stay as they are.  `rows`: for
 // kernels that copy whole row segments, a mask that is not contiguous in keys, or whose 16-bit rows
-// start off a dword (odd key counts), is laid out anew before it is broadcast (read element by
-// element instead, a layer of 2 x 32 heads x 2869 rows under such a mask took 2.26 ms; as float32 rows 0.89)
+// are not whole dwords from a dword on (odd key counts, also where the rows are a slice of even ones),
+// is laid out anew before it is broadcast (read element by element instead, a layer of 2 x 32 heads x
+// 2869 rows under such a mask took 2.26 ms; as float32 rows 0.89)
 Tensor attention_mask(const Checker& c, const c10::optional<Tensor>& mask_in, const Tensor& q_rot, int64_t sk,
                       bool own_type = false, bool rows = false) {
   if (!mask_in.has_value() || !mask_in->defined()) return Tensor();
@@ -164,7 +165,8 @@ Tensor attention_mask(const Checker& c, const c10::optional<Tensor>& mask_in, co
   while (mask.dim() < 4) mask = mask.unsqueeze(0);
   if (rows && mask.size(3) > 1) {
     if (mask.stride(3) != 1) mask = mask.contiguous();
-    const bool odd = ((mask.storage_offset() | mask.stride(0) | mask.stride(1) | mask.stride(2)) & 1) != 0;
+    const bool odd =
+        ((mask.storage_offset() | mask.stride(0) | mask.stride(1) | mask.stride(2) | mask.size(3)) & 1) != 0;
     if (mask.scalar_type() != at::kFloat && odd) mask = mask.to(at::kFloat).contiguous();
   }
   return mask.expand({q_rot.size(0), q_rot.size(1), q_rot.size(2), sk});
