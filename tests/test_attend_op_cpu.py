@@ -50,3 +50,24 @@ def test_attend_shape(mask):
 def test_attend_refuses(bad, match):
     with pytest.raises(RuntimeError, match=match):
         _args(**bad)
+
+
+@pytest.mark.parametrize("mdt", [torch.bfloat16, torch.float16, torch.float64, torch.bool])
+@pytest.mark.parametrize("few", [False, True])
+def test_mask_checks_convert_nothing(mdt, few):
+    """The checks look at a mask's shape only: a conversion belongs to the call that uses it, once
+    (tests/test_gpu_prefill_expanded.py counts those)."""
+    from torch.profiler import ProfilerActivity, profile
+
+    sq = 1 if few else SQ
+    m = _e(B, 1, sq, SK, dtype=mdt)
+    k = dict(q=_e(B, HQ, sq, D, dtype=torch.bfloat16), mask=m)
+    n = B * HKV * SK
+    with profile(activities=[ProfilerActivity.CPU]) as prof:
+        _args(**k)
+        ops().attention(_e(B, HQ, sq, D, dtype=F16), _e(B, HQ, sq, D), _e(n, 32, dtype=U8), _e(n, 16, dtype=U8),
+                        _e(n, dtype=F16), _e(n, dtype=F16), _e(4, dtype=F16), 3, _e(n, 48, dtype=U8), _e(n, dtype=F16),
+                        _e(8), 3, _e(2, D, D, dtype=F16), HKV, SK, 0, 0.01, 0.09, False, m, torch.float32, 1)
+    names = [e.name for e in prof.events()]
+    assert any("tq::attend" in x for x in names) and any("tq::attention" in x for x in names)
+    assert not [x for x in names if "_to_copy" in x or "contiguous" in x]

@@ -167,6 +167,26 @@ def test_prefill_masks_sliced_to_an_odd_key_count(d, mdt, rows):
     assert _err(_direct(q, kc, vc, ck, cv, mask=m), ref) < REL
 
 
+@pytest.mark.parametrize("mdt,dev", [(torch.float32, DEV), (torch.bfloat16, DEV), (torch.bool, DEV),
+                                     (torch.bfloat16, "cpu")])
+@pytest.mark.parametrize("sq", [1, 20])
+def test_masks_are_converted_once(mdt, dev, sq):
+    """Few-row and decode calls read float32 masks: what one `.to` to the device and that type does,
+    and no more."""
+    from torch.profiler import ProfilerActivity, profile
+
+    def copies(f):
+        f()
+        with profile(activities=[ProfilerActivity.CPU]) as prof:
+            f()
+        return sum(e.name == "aten::_to_copy" for e in prof.events())
+
+    kc, vc, q, ck, cv = _make(64, 3, 3, 4, 4, sq, 300)
+    m = torch.zeros(2, 1, sq, 300, device=dev, dtype=mdt)
+    assert (copies(lambda: compressed_attention(q, kc, vc, ck, cv, attention_mask=m))
+            == copies(lambda: m.to(q.device, torch.float32)))
+
+
 def test_prefill_rows_without_a_real_key():
     """A row whose mask is finfo.min everywhere attends all keys equally, as softmax does."""
     kc, vc, q, ck, cv = _make(128, 3, 3, 8, 2, 70, 100)

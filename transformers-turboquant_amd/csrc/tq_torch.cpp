@@ -149,17 +149,23 @@ void check_values(const Checker& c, const Tensor& q_rot, const Tensor& vcodes, c
   c.table(vpit, "split Pi_v^T", at::kHalf, 2 * D * D);
 }
 
-// the additive mask as a float32 view broadcast to [B, Hq, Sq, Sk] (no copy when it already
+// the mask broadcasts to [B, Hq, Sq, Sk] (metadata only: nothing is converted or copied)
+void check_mask(const Checker& c, const c10::optional<Tensor>& mask, const Tensor& q_rot, int64_t sk) {
+  if (!mask.has_value() || !mask->defined()) return;
+  TORCH_CHECK(mask->dim() <= 4, c.op, ": the mask must broadcast to [B, Hq, Sq, Sk], got ", mask->sizes());
+  mask->expand({q_rot.size(0), q_rot.size(1), q_rot.size(2), sk});
+}
+
+// a checked additive mask as a float32 view broadcast to [B, Hq, Sq, Sk] (no copy when it already
 // is float32 on the device); `own_type`: float16 and bfloat16 masks stay as they are.  `rows`: for
 // kernels that copy whole row segments, a mask that is not contiguous in keys, or whose 16-bit rows
 // are not whole dwords from a dword on (odd key counts, also where the rows are a slice of even ones),
 // is laid out anew before it is broadcast (read element by element instead, a layer of 2 x 32 heads x
 // 2869 rows under such a mask took 2.26 ms; as float32 rows 0.89)
-Tensor attention_mask(const Checker& c, const c10::optional<Tensor>& mask_in, const Tensor& q_rot, int64_t sk,
-                      bool own_type = false, bool rows = false) {
+Tensor attention_mask(const c10::optional<Tensor>& mask_in, const Tensor& q_rot, int64_t sk, bool own_type = false,
+                      bool rows = false) {
   if (!mask_in.has_value() || !mask_in->defined()) return Tensor();
   Tensor mask = *mask_in;
-  TORCH_CHECK(mask.dim() <= 4, c.op, ": the mask must broadcast to [B, Hq, Sq, Sk], got ", mask.sizes());
   const at::ScalarType type = own_type && is_act(mask.scalar_type()) ? mask.scalar_type() : at::kFloat;
   if (mask.device() != q_rot.device() || mask.scalar_type() != type) mask = mask.to(q_rot.device(), type);
   while (mask.dim() < 4) mask = mask.unsqueeze(0);
@@ -509,7 +515,7 @@ Tensor attention_meta(const Tensor& q_rot, const Tensor& q_proj, const Tensor& k
   TORCH_CHECK(is_act(out_dtype), c.op, ": out_dtype must be float32, float16 or bfloat16");
   check_prepared_keys(c, q_rot, q_proj, kcodes, ksigns, krn, kvn, kcent16, bits, hkv, sk, kv_stride);
   check_values(c, q_rot, vcodes, vvn, vcent32, val_bits, vpit, hkv, sk, kv_stride);
-  attention_mask(c, mask_in, q_rot, sk);  // broadcastable to [B, Hq, Sq, Sk]
+  check_mask(c, mask_in, q_rot, sk);
   return at::empty({q_rot.size(0), q_rot.size(2), q_rot.size(1), q_rot.size(3)}, q_rot.options().dtype(out_dtype));
 }
 
@@ -523,10 +529,9 @@ Tensor attention(const Tensor& q_rot, const Tensor& q_proj, const Tensor& kcodes
   // the checks, and the [B, Sq, Hq, D] output they return (allocated on q_rot's device)
   Tensor out = attention_meta(q_rot, q_proj, kcodes, ksigns, krn, kvn, kcent16, bits, vcodes, vvn, vcent32, val_bits,
                               vpit, hkv, sk, kv_stride, coeff, scale, causal, mask_in, out_dtype, workspace);
-  const Checker c{"tq::attention", q_rot.device()};
   const c10::DeviceGuard g(q_rot.device());
   const int64_t B = q_rot.size(0), Hq = q_rot.size(1), Sq = q_rot.size(2), D = q_rot.size(3);
-  Tensor mask = attention_mask(c, mask_in, q_rot, sk);
+  Tensor mask = attention_mask(mask_in, q_rot, sk);
   int64_t ms[4] = {0, 0, 0, 0};
   if (mask.defined())
     for (int i = 0; i < 4; ++i) ms[i] = mask.stride(i);
@@ -602,7 +607,7 @@ Tensor attend_meta(const Tensor& q, const Tensor& pi_split, const Tensor& s_eff1
   c.table(s_eff16, "f16 S_eff", at::kHalf, D * D);
   check_keys(c, q, kcodes, ksigns, krn, kvn, kcent16, bits, hkv, sk, kv_stride);
   check_values(c, q, vcodes, vvn, vcent32, val_bits, vpit, hkv, sk, kv_stride);
-  attention_mask(c, mask_in, q, sk, true);  // broadcastable to [B, Hq, Sq, Sk]
+  check_mask(c, mask_in, q, sk);
   return at::empty({q.size(0), q.size(2), q.size(1), D}, q.options().dtype(out_dtype));
 }
 
@@ -623,11 +628,10 @@ Tensor attend(const Tensor& q_in, const Tensor& pi_split, const Tensor& s_eff16,
   }
   Tensor out = attend_meta(q_in, pi_split, s_eff16, kcodes, ksigns, krn, kvn, kcent16, bits, vcodes, vvn, vcent32,
                            val_bits, vpit, hkv, sk, kv_stride, coeff, scale, causal, mask_in, out_dtype, workspace);
-  const Checker c{"tq::attend", q_in.device()};
   const c10::DeviceGuard g(q_in.device());
   Tensor q = activation(q_in);
   const int64_t B = q.size(0), Hq = q.size(1), Sq = q.size(2), D = q.size(3);
-  Tensor mask = attention_mask(c, mask_in, q, sk, true, true);
+  Tensor mask = attention_mask(mask_in, q, sk, true, true);
   int64_t ms[4] = {0, 0, 0, 0};
   if (mask.defined())
     for (int i = 0; i < 4; ++i) ms[i] = mask.stride(i);

@@ -178,6 +178,8 @@ class TurboQuantCacheLayer(CacheLayerMixin):
         tk, tv, need = self._gpu_room(key_compressor, val_compressor, k)
         if out_dtype not in (torch.float32, torch.float16, torch.bfloat16):
             out_dtype = torch.float32
+        if attention_mask is not None and attention_mask.device != k.device:
+            attention_mask = attention_mask.to(k.device, torch.float32)
         out = ops().cache_attend(
             k, v, q, tk.pi_split, tk.seff_split, tk.cent32, tk.bounds32, key_compressor.mse_bits, tv.pi_split,
             tv.bounds32, val_compressor.bits, tk.s_eff16, self.kp["packed_key_indices"], self.kp["packed_qjl_signs"],

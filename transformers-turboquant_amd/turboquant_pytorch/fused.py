@@ -74,6 +74,8 @@ def _attention_args(q: torch.Tensor, key_compressor, val_compressor, compressed_
     if scale is None:
         scale = 1.0 / math.sqrt(D)
     coeff = math.sqrt(math.pi / 2) / key_compressor.S.shape[0]
+    if attention_mask is not None and attention_mask.device != dev:
+        attention_mask = attention_mask.to(dev, torch.float32)
     mode = {"static": 2, True: 1, False: 0}[split_k]
     return tk, tv, (
         compressed_k["packed_key_indices"], compressed_k["packed_qjl_signs"], compressed_k["residual_norm"],
