@@ -187,6 +187,32 @@ def test_masks_are_converted_once(mdt, dev, sq):
             == copies(lambda: m.to(q.device, torch.float32)))
 
 
+@pytest.mark.parametrize("mdt,sk", [(torch.float32, 1100), (torch.bfloat16, 1101)])
+def test_broadcast_masks_are_laid_out_once(mdt, sk):
+    """A mask that the caller has expanded over batch and heads, and that has to be laid out anew
+    (not contiguous in keys; 16-bit rows of an odd key count), is copied without its repeats: the
+    call's memory grows by one [Sq, Sk] float32 plane (a second one while a 16-bit copy is converted),
+    not by B x Hq of them."""
+    d, sq, hq, hkv, B = 64, 100, 16, 4, 2
+    kc, vc, q, ck, cv = _make(d, 3, 3, hq, hkv, sq, sk)
+    g = torch.Generator(device=DEV).manual_seed(sk)
+    one = torch.randn(sk, sq, device=DEV, generator=g).to(mdt)
+    plain = one.t().contiguous()
+
+    def peak(m):
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        base = torch.cuda.memory_allocated()
+        out = compressed_attention(q, kc, vc, ck, cv, attention_mask=m)
+        return torch.cuda.max_memory_allocated() - base, out
+
+    bare, ref = peak(plain.float())
+    for m in (one.t().expand(B, hq, sq, sk), plain.expand(B, hq, sq, sk)):
+        used, out = peak(m)
+        assert torch.equal(out, ref)
+        assert used - bare <= 2 * 4 * sq * sk + 4096
+
+
 def test_prefill_rows_without_a_real_key():
     """A row whose mask is finfo.min everywhere attends all keys equally, as softmax does."""
     kc, vc, q, ck, cv = _make(128, 3, 3, 8, 2, 70, 100)

@@ -161,7 +161,8 @@ void check_mask(const Checker& c, const c10::optional<Tensor>& mask, const Tenso
 // kernels that copy whole row segments, a mask that is not contiguous in keys, or whose 16-bit rows
 // are not whole dwords from a dword on (odd key counts, also where the rows are a slice of even ones),
 // is laid out anew before it is broadcast (read element by element instead, a layer of 2 x 32 heads x
-// 2869 rows under such a mask took 2.26 ms; as float32 rows 0.89)
+// 2869 rows under such a mask took 2.26 ms; as float32 rows 0.89), without the repeats of dims that the
+// caller has already broadcast
 Tensor attention_mask(const c10::optional<Tensor>& mask_in, const Tensor& q_rot, int64_t sk, bool own_type = false,
                       bool rows = false) {
   if (!mask_in.has_value() || !mask_in->defined()) return Tensor();
@@ -170,6 +171,8 @@ Tensor attention_mask(const c10::optional<Tensor>& mask_in, const Tensor& q_rot,
   if (mask.device() != q_rot.device() || mask.scalar_type() != type) mask = mask.to(q_rot.device(), type);
   while (mask.dim() < 4) mask = mask.unsqueeze(0);
   if (rows && mask.size(3) > 1) {
+    for (int i = 0; i < 3; ++i)
+      if (mask.stride(i) == 0 && mask.size(i) > 1) mask = mask.narrow(i, 0, 1);
     if (mask.stride(3) != 1) mask = mask.contiguous();
     const bool odd =
         ((mask.storage_offset() | mask.stride(0) | mask.stride(1) | mask.stride(2) | mask.size(3)) & 1) != 0;
