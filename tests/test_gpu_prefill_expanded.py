@@ -19,6 +19,7 @@ import torch
 
 from transformers_turboquant import TurboQuantCache
 from turboquant_pytorch import _native, compressed_attention
+from turboquant_pytorch.fused import attention_from_prepared
 from turboquant_pytorch.compressors import TurboQuantCompressorMSE, TurboQuantCompressorV2, _tables
 
 pytestmark = pytest.mark.gpu
@@ -211,6 +212,35 @@ def test_broadcast_masks_are_laid_out_once(mdt, sk):
         used, out = peak(m)
         assert torch.equal(out, ref)
         assert used - bare <= 2 * 4 * sq * sk + 4096
+
+
+@pytest.mark.parametrize("d,bits,vbits,hq,hkv,sq,sk", [
+    (64, 3, 3, 4, 4, 65, 1100),    # the packed path splits these over keys on its tiled kernel, although
+    (64, 4, 4, 12, 6, 64, 1100),   # it has a prefill kernel for the bit widths
+    (64, 2, 2, 4, 4, 128, 5000),
+    (128, 3, 2, 4, 2, 64, 700),    # no prefill kernel for the bit widths, or for the head dim
+    (80, 3, 3, 4, 2, 64, 700),
+])
+def test_weights_keep_their_lo_parts(d, bits, vbits, hq, hkv, sq, sk):
+    """Where the packed path keeps the softmax weights as f16 hi + lo, so does the expanded one.  Zero
+    queries make the weights the softmax of the mask alone; against V^ = f16(C_v vn) what is left is
+    the weights' own error (2^-22, one f16 would leave 2e-4), their f32 sums and exponents (a few 1e-7
+    each) and the hi + lo output rotation: below 1e-5 by a factor of three."""
+    print("case:", d, bits, vbits, hq, hkv, sq, sk, flush=True)
+    kc, vc, q, ck, cv = _make(d, bits, vbits, hq, hkv, sq, sk)
+    q = torch.zeros_like(q)
+    m = 2 * torch.randn(2, 1, sq, sk, device=DEV, generator=torch.Generator(device=DEV).manual_seed(d))
+    n = 2 * hkv * sk
+    vh = vc.centroids.float()[_unpack(cv["packed_indices"].reshape(n, -1), vc.bits, d)]
+    vh = (vh * cv["vec_norms"].float().reshape(n, 1)).half().double()
+    vh = vh.reshape(2, hkv, sk, d).repeat_interleave(hq // hkv, dim=1)
+    ref = ((torch.softmax(m.double(), -1).expand(2, hq, sq, sk) @ vh) @ vc.Pi.double()).transpose(1, 2)
+    q_rot, q_proj = kc.prepare_queries(q)
+    errs = [_err(x, ref) for x in (attention_from_prepared(q_rot, q_proj, kc, vc, ck, cv, attention_mask=m),
+                                   compressed_attention(q, kc, vc, ck, cv, attention_mask=m),
+                                   _direct(q, kc, vc, ck, cv, mask=m))]
+    print("errors: packed %.2e, expanded %.2e, expanded through the C entry %.2e" % tuple(errs), flush=True)
+    assert max(errs) < 1e-5
 
 
 def test_prefill_rows_without_a_real_key():

@@ -921,6 +921,20 @@ static int check_common(const char* what, int32_t B, int32_t Hq, int32_t Hkv, in
   return TQ_OK;
 }
 
+// Whether tq_attention_fwd_kv runs the prefill kernel, which keeps the softmax weights as one f16
+// (the tiled kernel keeps f16 hi + lo); split: with keys split over blocks, one query block per kv head
+static bool prefill_runs(bool split, int Hq, int Hkv, int Sq, int d, int bits, int val_bits, bool masked) {
+  return split ? prefill_split_applies(Hq, Hkv, Sq, d, bits, val_bits, masked)
+               : prefill_applies(Hq, Hkv, d, bits, val_bits, masked);
+}
+
+namespace tq {
+// the same of a call that has its whole workspace: the expanded-key kernels keep the weights as it does
+bool weights_are_f16(int B, int Hq, int Hkv, int Sq, int Sk, int d, int bits, int val_bits, bool masked) {
+  return prefill_runs(tiled_split_plan(B, Hq, Hkv, Sq, Sk, d).nsplit > 0, Hq, Hkv, Sq, d, bits, val_bits, masked);
+}
+}  // namespace tq
+
 // the tiled kernel serves GQA groups of at most block_rows(d, scores) query heads
 static int check_group(const char* what, int32_t Hq, int32_t Hkv, int32_t d, bool scores) {
   TQ_REQUIRE(Hq / Hkv <= block_rows(d, scores), "%s: group size %d exceeds %d at head_dim %d", what,
@@ -1035,7 +1049,8 @@ int tq_attention_fwd_kv(const uint16_t* q_rot, const float* q_proj, const uint8_
     return merge_key_splits(part_o, part_ml, val_pit_split, B, Hq, Hkv, Sq, C, sp.nsplit, d, out, out_dtype, sob,
                             soh, sos, as_stream(stream));
   };
-  if (split && prefill_split_applies(Hq, Hkv, Sq, d, bits, val_bits, mask != nullptr)) {
+  const bool prefill = prefill_runs(split, Hq, Hkv, Sq, d, bits, val_bits, mask != nullptr);
+  if (split && prefill) {
     // head_dim 64 / 128: the prefill kernel split over keys
     const int C = (Hq / Hkv) * Sq;
     float* part_o = static_cast<float*>(workspace);
@@ -1047,7 +1062,7 @@ int tq_attention_fwd_kv(const uint16_t* q_rot, const float* q_proj, const uint8_
     if (st != TQ_OK) return st;
     return merge_split(part_o, part_ml, C);
   }
-  if (!split && prefill_applies(Hq, Hkv, d, bits, val_bits, mask != nullptr))
+  if (prefill)
     return prefill_attention(ldk, q_rot, q_proj, key_codes, key_signs, key_rn, key_vn, key_centroids_f16, bits,
                              val_codes, val_vn, val_centroids, val_pit_split, B, Hq, Hkv, Sq, Sk, d, coeff, scale,
                              causal, mask, smb, smh, smq, smk, out, out_dtype, sob, soh, sos, as_stream(stream));

@@ -1264,7 +1264,8 @@ static DensePlan dense_plan(int64_t groups, int G, int Sq, int Sk, int d, bool c
   return best;
 }
 
-bool prefill_applies(int Hq, int Hkv, int d, int bits, int val_bits, bool masked);  // tq_prefill.hip
+// tq_attn.hip
+bool weights_are_f16(int B, int Hq, int Hkv, int Sq, int Sk, int d, int bits, int val_bits, bool masked);
 
 }  // namespace tq
 
@@ -1388,9 +1389,9 @@ int tq_prefill_attention(const void* q, int32_t dtype, int64_t sqb, int64_t sqh,
   uint16_t* seff_frag = static_cast<uint16_t*>(workspace);
   uint16_t* q_rot = seff_frag + static_cast<int64_t>(DP) * DP;
   launch_rotate(q, dtype, B, Hq, Sq, d, sqb, sqh, sqs, key_pi_split, key_s_eff_f16, q_rot, seff_frag, cus, s);
-  // P as f16 (hi, lo) where the term-by-term path keeps it so (its tiled kernel); one f16 where its
-  // prefill kernel rounds it
-  const bool plo = !prefill_applies(Hq, Hkv, d, bits, val_bits, mask != nullptr);
+  // P as f16 (hi, lo) where the term-by-term path keeps it so (its tiled kernel, split over keys or
+  // not); one f16 where the kernel it would run for this shape rounds it (the prefill kernel)
+  const bool plo = !weights_are_f16(B, Hq, Hkv, Sq, Sk, d, bits, val_bits, mask != nullptr);
   const int width = row_width(d, reinterpret_cast<uintptr_t>(key_codes) | reinterpret_cast<uintptr_t>(key_signs) |
                                      reinterpret_cast<uintptr_t>(val_codes));
   uint8_t* tiles = static_cast<uint8_t*>(workspace) + qbytes;
