@@ -20,6 +20,7 @@ import torch
 from transformers_turboquant import TurboQuantCache
 from turboquant_pytorch import _native, compressed_attention
 from turboquant_pytorch.fused import attention_from_prepared
+from turboquant_pytorch.kernels.attention import scores_from_prepared
 from turboquant_pytorch.compressors import TurboQuantCompressorMSE, TurboQuantCompressorV2, _tables
 
 pytestmark = pytest.mark.gpu
@@ -241,6 +242,67 @@ def test_weights_keep_their_lo_parts(d, bits, vbits, hq, hkv, sq, sk):
                                    _direct(q, kc, vc, ck, cv, mask=m))]
     print("errors: packed %.2e, expanded %.2e, expanded through the C entry %.2e" % tuple(errs), flush=True)
     assert max(errs) < 1e-5
+
+
+@pytest.mark.parametrize("d,hq,hkv,sq,sk,masked", [
+    (128, 8, 2, 70, 140, False), (128, 8, 2, 70, 1100, True), (128, 8, 8, 300, 1200, False),
+    (64, 8, 2, 70, 1100, True), (64, 4, 4, 200, 200, False), (80, 8, 2, 40, 700, False), (80, 8, 2, 40, 700, True),
+    (200, 4, 4, 70, 90, False),
+])
+def test_norms_that_are_not_finite(d, hq, hkv, sq, sk, masked):
+    """A key whose f16 norm overflowed has scores of +-inf: no weight in the rows where it is -inf, NaN
+    in the rows where it is +inf.  Neither the rows that do not attend it nor the other keys of its tile
+    see any of it.  Row for row as on the packed path, whose score terms carry the norms apart."""
+    print("case:", d, hq, hkv, sq, sk, masked, flush=True)
+    kc, vc, q, ck, cv = _make(d, 3, 3, hq, hkv, sq, sk)
+    g = torch.Generator(device=DEV).manual_seed(d)
+    mask = None
+    if masked:
+        mask = torch.randn(2, 1, sq, sk, device=DEV, generator=g)
+        mask[0, :, :, : sk // 3] = torch.finfo(torch.float32).min
+    inf, nan, last = math.inf, math.nan, sk - sq // 2  # a key that the first half of the causal rows misses
+    q_rot, q_proj = kc.prepare_queries(q)
+    vn, rn = ck["vec_norms"], ck["residual_norm"]
+    for head, key, v, r in ((0, last, inf, 1.0), (0, 3, 1e-4, 1e-5), (1, last, inf, inf), (2, last, 1.0, inf),
+                            (3, last, nan, 1.0), (2, 5, inf, 1.0)):
+        at = (head % (2 * hkv)) * sk + key
+        vn.view(-1)[at], rn.view(-1)[at] = v, r
+    want = attention_from_prepared(q_rot, q_proj, kc, vc, ck, cv, attention_mask=mask, causal=True)
+    bad = torch.isnan(want)
+    assert 0.05 < bad.float().mean() < 0.95  # rows of both kinds
+    for got in (compressed_attention(q, kc, vc, ck, cv, attention_mask=mask, causal=True),
+                _direct(q, kc, vc, ck, cv, mask=mask, causal=True)):
+        assert torch.equal(torch.isnan(got), bad)
+        assert _err(got[~bad], want[~bad].double()) < REL
+
+
+@pytest.mark.parametrize("d,sq,sk", [(128, 64, 96), (64, 140, 75), (80, 140, 64), (256, 140, 96)])
+def test_expanded_scores_over_all_norms(d, sq, sk):
+    """Every key's scores at f32 grade whatever its neighbours' norms (f16's whole range in a tile), and
+    the infinities and NaNs of the packed path.  Per key: a key's rounding flips of q_rot (see
+    test_expanded_scores) are a sum over sq rows here, so the bar of 2e-5 is four times that of a matrix.
+    The sign of an infinity is a dot product's: where that is within its rounding of 0 (one part in 2^12
+    of its size: less than a thousandth of them) it can fall either way."""
+    kc, _, q, ck, _ = _make(d, 3, 3, 8, 2, sq, sk, scale=lambda n: 10 ** torch.linspace(
+        -4, 3, n, device=DEV)[torch.randperm(n, device=DEV, generator=torch.Generator(device=DEV).manual_seed(n))][:, None])
+    q_rot, q_proj = kc.prepare_queries(q)
+    t = _tables(kc, q.device, True)
+    args = (ck["packed_key_indices"], ck["packed_qjl_signs"], ck["residual_norm"], ck["vec_norms"], t.cent16, 3,
+            math.sqrt(math.pi / 2) / d, 2, sk, sk)
+    want = scores_from_prepared(q_rot, q_proj, *args).double()
+    assert torch.isfinite(want).all()
+    got = kc.asymmetric_attention_scores(q, ck)
+    err = (got.double() - want).norm(dim=2) / want.norm(dim=2)  # per (batch, head, key)
+    print("largest error of a key: %.2e" % err.max().item(), flush=True)
+    assert err.max() < 8e-5
+    for key, v, r in ((1, math.inf, 1.0), (34, 1.0, math.inf), (40, math.inf, math.inf), (sk - 1, math.nan, 1.0)):
+        for plane, x in (("vec_norms", v), ("residual_norm", r)):
+            ck[plane].view(-1, sk)[:, key] = x
+    want, got = scores_from_prepared(q_rot, q_proj, *args), kc.asymmetric_attention_scores(q, ck)
+    fin = torch.isfinite(want)
+    assert torch.equal(torch.isfinite(got), fin)
+    assert (got.nan_to_num(0, 1, -1) != want.nan_to_num(0, 1, -1))[~fin].float().mean() < 1e-3
+    assert _err(got[fin], want[fin].double()) < 2e-5
 
 
 def test_prefill_rows_without_a_real_key():

@@ -16,8 +16,10 @@
 // v_mfma_f32_32x32x16_f16 A operand in lane order (16 bytes per lane), so that the attention
 // kernel copies records into LDS as they are and reads fragments at lane * 16: contiguous in
 // memory, free of bank conflicts, no address arithmetic.  k^ carries a power of two per tile
-// (from a bound on the tile's largest |k^|), whose inverse the score scaling takes, so that
-// neither hi nor lo leaves f16's normal range at any key norm.
+// (from a bound on the tile's largest |k^|), whose inverse the score scaling takes: hi stays finite
+// and lo a normal f16 for keys down to kMixed of that bound.  A tile with a smaller key, or with a
+// norm that is not finite, is a mixed tile: its keys carry factors of their own, one for the hi and
+// one for the lo product, and the kernels take its scores over a separate, slower branch.
 //
 // Bound and measurements (bits 3, 32 / 8 heads, head_dim 128, against tq_query_prep and the
 // term-by-term prefill kernel, one MI355X): 8192 causal rows 1160 -> 815 us for the whole layer,
@@ -61,6 +63,8 @@ __device__ __forceinline__ half8 mat8(const uint16_t* m, int i, int j, int d) {
 }
 
 constexpr int kDenseKeys = 32;  // keys per tile
+constexpr float kMixed = 0x1p-11f;  // keys below this part of their tile's bound make it a mixed tile
+constexpr int kKeyFac = 2 * kDenseKeys;  // floats of a mixed tile's factors: (hi, lo) per key
 template <int DP, bool VALS = true>
 constexpr int dense_rec() { return (VALS ? 3 : 2) * DP * 64; }  // bytes of a tile record; keys only without VALS
 
@@ -221,7 +225,7 @@ struct ExpandArgs {
   int64_t ldk, bh0, total;   // total: tiles of this launch
   float coeff;
   uint8_t* tiles;
-  float* tfac;
+  float *tfac, *kfac;  // factor of each tile (0: a mixed tile); key factors of mixed tiles
 };
 
 // A row's bits of 32 dims, b <= 4 bits each, as dwords (dims past d read as code 0)
@@ -288,7 +292,7 @@ __global__ void __launch_bounds__(2 * DP) dense_expand_kernel(ExpandArgs a) {
   asum = wave_max(asum);
   if (lane == 0) s_bound[w] = asum;
   __syncthreads();
-  float smax = 0.f, cmax = 0.f;
+  float smax = 0.f, cmax = 0.f;  // |S_eff^T s| and |C| of any key
 #pragma unroll
   for (int i = 0; i < NW; ++i) smax = fmaxf(smax, s_bound[i]);
 #pragma unroll
@@ -341,10 +345,24 @@ __global__ void __launch_bounds__(2 * DP) dense_expand_kernel(ExpandArgs a) {
     }
     // power-of-two tile scale: the bound vn cmax + |coeff| rn smax of the tile's largest |k^| lands
     // in [2^13, 2^14)
-    const float bound = wave_max(vn) * cmax + wave_max(fabsf(rn)) * smax;
-    const float up = qproj_split_scale(bound);
-    if (tid == 0) a.tfac[T] = 1.f / up;
+    const float bound = wave_max(fabsf(vn)) * cmax + wave_max(fabsf(rn)) * smax;
+    const float own = fabsf(vn) * cmax + fabsf(rn) * smax;  // this key's bound
+    const bool finite = own <= 3.0e38f;
+    const bool mixed = __any(own != 0.f && !(finite && own >= bound * kMixed));  // the same for every wave
+    float up = qproj_split_scale(bound);
+    if (tid == 0) a.tfac[T] = mixed ? 0.f : 1.f / up;
     uint8_t* rec = a.tiles + T * dense_rec<DP, VALS>();
+    if (mixed) {  // a key of finite norms takes a power of two of its own
+      asm volatile("; mixed tile" ::: "memory");
+      int e;
+      frexpf(own, &e);
+      up = finite && own > 0.f ? ldexpf(1.f, 14 - e) : 1.f;
+      if (tid < kDenseKeys) {  // lanes (key tid, h 0) of wave 0
+        float* f = a.kfac + T * kKeyFac + 2 * tid;
+        f[0] = finite ? 1.f / up : vn;
+        f[1] = finite ? 1.f / up : rn;
+      }
+    }
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       const bool real = 32 * w + 16 * s + 8 * h < d;  // this lane's 8 dims
@@ -360,6 +378,25 @@ __global__ void __launch_bounds__(2 * DP) dense_expand_kernel(ExpandArgs a) {
       }
       *reinterpret_cast<half8*>(rec + (2 * w + s) * 1024 + lane * 16) = hi;
       *reinterpret_cast<half8*>(rec + (KS + 2 * w + s) * 1024 + lane * 16) = lo;
+    }
+    if (mixed && !finite) {
+      // infinite (or NaN) norms: the two terms apart, C in hi and S_eff^T s (one f16: only its sign
+      // matters) in lo.  The norms are the key's factors and enter with the scores, as the packed kernels
+      // have it: a score of +-inf
+      asm volatile("; norms not finite" ::: "memory");
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const bool real = 32 * w + 16 * s + 8 * h < d;
+        half8 hi, lo;
+        const uint32_t c = kf.codes8(2 * s + h, a.kb);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          hi[e] = static_cast<_Float16>(real ? s_kc[(c >> (a.kb * e)) & km] : 0.f);
+          lo[e] = static_cast<_Float16>(real ? acc[8 * s + e] : 0.f);
+        }
+        *reinterpret_cast<half8*>(rec + (2 * w + s) * 1024 + lane * 16) = hi;
+        *reinterpret_cast<half8*>(rec + (KS + 2 * w + s) * 1024 + lane * 16) = lo;
+      }
     }
     if constexpr (VALS) {
       // V^ into row perm32 of the block
@@ -397,7 +434,7 @@ __global__ void __launch_bounds__(2 * DP) dense_expand_kernel(ExpandArgs a) {
 struct DenseArgs {
   const uint16_t* q_rot;
   const uint8_t* tiles;
-  const float* tfac;
+  const float *tfac, *kfac;
   const uint16_t* vpit;  // split Pi_v^T (hi, lo), [2][d][d]
   int Hq, Hkv, Sq, Sk, d, G, QT, nqb, nbh, ntile;
   int64_t bh0;
@@ -618,7 +655,7 @@ dense_attn_kernel(DenseArgs a) {
   // this wave's tiles end at tw (its last row's last key); tiles from tf on need masking, tiles before
   // tfb in no wave of the block.  A wave without columns (tw = tb) only copies
   int tw = te, tf = te;
-  const int tfb = min(te, (a.causal ? min(qblk * a.QT + off + 1, a.Sk) : a.Sk) / kDenseKeys);
+  int tfb = min(te, (a.causal ? min(qblk * a.QT + off + 1, a.Sk) : a.Sk) / kDenseKeys);
   {
     const int ql0 = wave * 32 / a.G, ql1 = min((wave * 32 + 31) / a.G, a.QT - 1);
     const int i0 = qblk * a.QT + ql0, i1 = min(qblk * a.QT + ql1, a.Sq - 1);
@@ -660,6 +697,7 @@ dense_attn_kernel(DenseArgs a) {
   // ---- ring
   const uint8_t* recs = a.tiles + static_cast<int64_t>(blk.bhi) * a.ntile * REC;
   const float* tfac = a.tfac + static_cast<int64_t>(blk.bhi) * a.ntile;
+  const float* kfac = a.kfac + static_cast<int64_t>(blk.bhi) * a.ntile * kKeyFac;
   const uint32_t ring_lds = lds_offset(ring);
   // copy the next tile's record into the ring; past the last tile the last one again (into a free
   // slot), so that every iteration has the same number of copies in flight.  The descriptor and the
@@ -704,6 +742,10 @@ dense_attn_kernel(DenseArgs a) {
   auto factor = [&](int t) __attribute__((always_inline)) {
     return fa * __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, fv), (t - tb) & 63));
   };
+  auto mixed_tile = [&](int t) __attribute__((always_inline)) {
+    return __builtin_amdgcn_readlane(__builtin_bit_cast(int, fv), (t - tb) & 63) == 0;
+  };
+  bool mixed = false;  // the block meets a mixed tile
   auto frag = [&](const uint8_t* rec, int f) __attribute__((always_inline)) {  // rec: record + lane * 16
     return *reinterpret_cast<const half8*>(rec + f * 1024);
   };
@@ -800,6 +842,23 @@ dense_attn_kernel(DenseArgs a) {
     return max_raw(max8_raw(sc[0], sc[1], sc[2], sc[3], sc[4], sc[5], sc[6], sc[7]),
                    max8_raw(sc[8], sc[9], sc[10], sc[11], sc[12], sc[13], sc[14], sc[15]));
   };
+  // scores of a mixed tile t (landed at `rec`): hi and lo products under their keys' own factors
+  auto mixed_scores = [&](int t, const uint8_t* rec) __attribute__((always_inline)) {
+    asm volatile("; mixed tile" ::: "memory");  // fragments are read anew: none is kept for this branch
+    float16v sh = zero16(), sl = zero16();
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      sh = mfma32x32x16(frag(rec, ks), qf[ks], sh);
+      sl = mfma32x32x16(frag(rec, KS + ks), qf[ks], sl);
+    }
+    const float* kf = kfac + static_cast<int64_t>(t) * kKeyFac + 8 * h;
+#pragma unroll
+    for (int i = 0; i < 16; i += 2) {  // keys 8 (i / 4) + 4 h + i % 4, + 1
+      const float4v k2 = *reinterpret_cast<const float4v*>(kf + 16 * (i >> 2) + 2 * (i & 3));
+      sc[i] = score_at(fmaf(sl[i], k2[1], sh[i] * k2[0]), i, fa);
+      sc[i + 1] = score_at(fmaf(sl[i + 1], k2[3], sh[i + 1] * k2[2]), i + 1, fa);
+    }
+  };
   // scores of tile t (landed at `rec`) with nothing to overlap: the first tile
   auto first_scores = [&](int t, const uint8_t* rec) __attribute__((always_inline)) {
     float16v s = zero16();
@@ -809,6 +868,7 @@ dense_attn_kernel(DenseArgs a) {
     const float f = factor(t);
 #pragma unroll
     for (int i = 0; i < 16; ++i) sc[i] = score_at(s[i], i, f);
+    if (mixed && mixed_tile(t)) mixed_scores(t, rec);
     if (t >= tf) clip_edge(t);
     settle(max16());
   };
@@ -877,7 +937,15 @@ dense_attn_kernel(DenseArgs a) {
     });
   };
 
-  factors(tb);  // and waits for q: the ring's waits count copies only
+  // A block with a mixed tile takes every tile as one that needs masking: the loops before that one know
+  // nothing of mixed tiles.  (A tile's factor is 1/6000 of its record.)
+  fv = tfac[min(tb + lane, te - 1)];
+  float least = fv;
+#pragma unroll 4
+  for (int t = tb + 64; t < te; t += 64) least = fminf(least, tfac[min(t + lane, te - 1)]);
+  mixed = __any(least == 0.f);
+  if (mixed) tf = tfb = tb;
+  wait_vm0_visible();  // q and the factors have landed: the ring's waits count copies only
   if (te > tb) {
 #pragma unroll
     for (int i = 0; i < LEAD; ++i) {
@@ -941,6 +1009,7 @@ dense_attn_kernel(DenseArgs a) {
       const uint8_t* nxt = next(cur);
       if (t + 1 < tw) {
         tile(t, cur, nxt, std::true_type{});
+        if (mixed && mixed_tile(t + 1)) mixed_scores(t + 1, nxt);
         clip_edge(t + 1);
         settle(max16());
       } else if (t < tw) {
@@ -1074,7 +1143,7 @@ __global__ void __launch_bounds__(2 * DP) dense_merge_kernel(DenseArgs a, int nw
 struct DenseScoreArgs {
   const uint16_t* q_rot;
   const uint8_t* tiles;  // keys only
-  const float* tfac;
+  const float *tfac, *kfac;
   int Hq, Hkv, Sq, Sk, d, G, rchunks, nbh, ntile, nblk, cpt;  // rchunks: 32-row chunks of a head
   int64_t bh0;
   float* out;  // [B, Hq, Sq, Sk]
@@ -1119,6 +1188,7 @@ __global__ void __launch_bounds__(256) dense_scores_kernel(DenseScoreArgs a) {
   // rows past the head's end are dropped by the store's range check
   const rsrc_t ro = make_rsrc(a.out + row0 * a.Sk, live ? static_cast<uint32_t>(rows) * a.Sk * 4 : 0);
   const float* tfac = a.tfac + static_cast<int64_t>(bhi) * a.ntile;
+  const float* kfac = a.kfac + static_cast<int64_t>(bhi) * a.ntile * kKeyFac;
   float fv = 0.f;
   auto factors = [&](int t) __attribute__((always_inline)) {  // of tiles t .. t + 63
     fv = tfac[min(t + lane, te - 1)];
@@ -1159,7 +1229,21 @@ __global__ void __launch_bounds__(256) dense_scores_kernel(DenseScoreArgs a) {
       s = mfma32x32x16(qf[ks], *reinterpret_cast<const half8*>(rec + ks * 1024), s);
       s = mfma32x32x16(qf[ks], *reinterpret_cast<const half8*>(rec + (KS + ks) * 1024), s);
     }
-    const float f = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, fv), (t - tb) & 63));
+    float f = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, fv), (t - tb) & 63));
+    if (__builtin_expect(f == 0.f, 0)) {  // a mixed tile: hi and lo apart, under this lane's key's factors
+      asm volatile("; mixed tile" ::: "memory");  // fragments read anew: none is kept for this branch
+      float16v sl = zero16();
+      s = zero16();
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        s = mfma32x32x16(qf[ks], *reinterpret_cast<const half8*>(rec + ks * 1024), s);
+        sl = mfma32x32x16(qf[ks], *reinterpret_cast<const half8*>(rec + (KS + ks) * 1024), sl);
+      }
+      const float* kf = kfac + static_cast<int64_t>(t) * kKeyFac + 2 * n;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[i] = fmaf(sl[i], kf[1], s[i] * kf[0]);
+      f = 1.f;
+    }
     const int key = t * kDenseKeys + n;
     // the range check covers the lane offset: it carries the row, and keys past Sk start out of range
     // (Sk < 2^24: neither wraps)
@@ -1259,7 +1343,8 @@ static DensePlan dense_plan(int64_t groups, int G, int Sq, int Sk, int d, bool c
     }
   }
   const int64_t recs = static_cast<int64_t>(best.nqb) * best.nsplit * best.NW;
-  best.group_bytes = (static_cast<int64_t>(ntile) * 4 + 15) / 16 * 16 + static_cast<int64_t>(ntile) * (3 * DP * 64) +
+  best.group_bytes = (static_cast<int64_t>(ntile) * 4 + 15) / 16 * 16 +
+                     static_cast<int64_t>(ntile) * (3 * DP * 64 + kKeyFac * 4) +
                      (best.nsplit > 1 ? recs * (DP * 32 + 64) * 4 : 0);
   return best;
 }
@@ -1282,10 +1367,10 @@ static int64_t dense_q_bytes(int B, int Hq, int Sq, int d) {
   return 2 * DP * DP + (static_cast<int64_t>(B) * Hq * Sq * d * 2 + 255) / 256 * 256;
 }
 
-// workspace of one (batch, kv head)'s expanded keys and tile factors
+// workspace of one (batch, kv head)'s expanded keys and factors
 static int64_t score_group_bytes(int Sk, int d) {
   const int64_t nt = (Sk + kDenseKeys - 1) / kDenseKeys;
-  return nt * (2 * pad_dim(d) * 64) + (nt * 4 + 15) / 16 * 16;
+  return nt * (2 * pad_dim(d) * 64 + kKeyFac * 4) + (nt * 4 + 15) / 16 * 16;
 }
 
 // Bytes per load that every packed row (d / 8 bytes per code bit) and plane base allows the expansion
@@ -1397,7 +1482,8 @@ int tq_prefill_attention(const void* q, int32_t dtype, int64_t sqb, int64_t sqh,
   uint8_t* tiles = static_cast<uint8_t*>(workspace) + qbytes;
   float* part_o = reinterpret_cast<float*>(tiles + per * p.ntile * (3 * DP * 64));
   float* part_ml = part_o + (p.nsplit > 1 ? per * recs * DP * 32 : 0);
-  float* tfac = part_ml + (p.nsplit > 1 ? per * recs * 64 : 0);
+  float* kfac = part_ml + (p.nsplit > 1 ? per * recs * 64 : 0);
+  float* tfac = kfac + per * p.ntile * kKeyFac;
   for (int64_t g0 = 0; g0 < groups; g0 += per) {
     const int nbh = static_cast<int>(std::min(per, groups - g0));
     ExpandArgs e{};
@@ -1406,9 +1492,9 @@ int tq_prefill_attention(const void* q, int32_t dtype, int64_t sqb, int64_t sqh,
     e.vcent = val_centroids;
     e.Sk = Sk; e.d = d; e.kb = bits - 1; e.vb = val_bits; e.ntile = p.ntile;
     e.ldk = ldk; e.bh0 = g0; e.total = static_cast<int64_t>(nbh) * p.ntile;
-    e.coeff = coeff; e.tiles = tiles; e.tfac = tfac;
+    e.coeff = coeff; e.tiles = tiles; e.tfac = tfac; e.kfac = kfac;
     DenseArgs a{};
-    a.q_rot = q_rot; a.tiles = tiles; a.tfac = tfac; a.vpit = val_pit_split;
+    a.q_rot = q_rot; a.tiles = tiles; a.tfac = tfac; a.kfac = kfac; a.vpit = val_pit_split;
     a.Hq = Hq; a.Hkv = Hkv; a.Sq = Sq; a.Sk = Sk; a.d = d; a.G = G; a.QT = p.QT; a.nqb = p.nqb; a.nbh = nbh;
     a.ntile = p.ntile; a.bh0 = g0; a.scale = scale; a.causal = causal;
     a.mask = mask; a.mask_dtype = mask_dtype; a.smb = smb; a.smh = smh; a.smq = smq; a.smk = smk;
@@ -1506,7 +1592,9 @@ int tq_prefill_scores(const void* q, int32_t dtype, int64_t sqb, int64_t sqh, in
   TQ_REQUIRE(static_cast<int64_t>(G) * a.rchunks < (int64_t(1) << 31) && groups < (int64_t(1) << 31), "%s: too many rows",
              what);
   a.nblk = (G * a.rchunks + 3) / 4;
-  a.tfac = reinterpret_cast<float*>(tiles + per * a.ntile * static_cast<int64_t>(2 * DP * 64));
+  float* kfac = reinterpret_cast<float*>(tiles + per * a.ntile * static_cast<int64_t>(2 * DP * 64));
+  float* tfac = kfac + per * a.ntile * kKeyFac;
+  a.kfac = kfac; a.tfac = tfac;
   // about eight blocks per compute unit, of at least four tiles
   const int64_t blocks = std::min(per, groups) * a.nblk;
   a.cpt = static_cast<int>(std::min<int64_t>(a.ntile, std::max<int64_t>(4, blocks * a.ntile / (8LL * cus))));
@@ -1519,7 +1607,7 @@ int tq_prefill_scores(const void* q, int32_t dtype, int64_t sqb, int64_t sqh, in
     e.kcodes = key_codes; e.ksigns = key_signs; e.krn = key_rn; e.kvn = key_vn; e.kcent = key_centroids_f16;
     e.seff_frag = seff_frag; e.Sk = Sk; e.d = d; e.kb = bits - 1; e.vb = 1; e.ntile = a.ntile;
     e.ldk = ldk; e.bh0 = g0; e.total = static_cast<int64_t>(a.nbh) * a.ntile;
-    e.coeff = coeff; e.tiles = tiles; e.tfac = const_cast<float*>(a.tfac);
+    e.coeff = coeff; e.tiles = tiles; e.tfac = tfac; e.kfac = kfac;
     const unsigned egrid = static_cast<unsigned>(std::min<int64_t>(e.total, 8LL * cus));
     const unsigned grid = static_cast<unsigned>(a.nbh) * a.nblk * nsplit;
 #define TQ_SCORES_CASE(DD)                                                                     \
