@@ -305,6 +305,33 @@ def test_expanded_scores_over_all_norms(d, sq, sk):
     assert _err(got[fin], want[fin].double()) < 2e-5
 
 
+@pytest.mark.parametrize("B,d,hq,hkv,sq,sk,masked,expanded", [
+    (1, 128, 32, 8, 64, 600, False, True),      # few long query blocks
+    (1, 128, 32, 8, 32, 600, False, False),     # 128 columns: the packed kernel splits the keys
+    (24, 128, 12, 12, 132, 2000, False, False),  # many sequences fill the packed kernel's grid
+    (2, 128, 12, 12, 132, 2000, False, True),
+    (48, 64, 12, 12, 64, 500, False, False),
+    (1, 64, 12, 12, 63, 200, False, False),     # below 64 columns
+    (8, 64, 12, 12, 64, 1100, True, False),     # under a mask: 64 columns are one block
+    (8, 64, 12, 12, 65, 1100, True, True),      # the tiled kernel's split
+    (48, 64, 12, 12, 96, 1500, True, False),
+    (1, 128, 32, 8, 40, 900, True, True),
+    (1, 80, 32, 32, 64, 300, False, True),      # no prefill kernel
+])
+def test_prefill_route(B, d, hq, hkv, sq, sk, masked, expanded):
+    """Which kernels a call takes, on both sides of each line of the rule: bit for bit those of the path
+    named here, and in agreement with the other path."""
+    print("case:", B, d, hq, hkv, sq, sk, masked, expanded, flush=True)
+    kc, vc, q, ck, cv = _make(d, 3, 3, hq, hkv, sq, sk, B=B)
+    m = torch.randn(B, 1, sq, sk, device=DEV, generator=torch.Generator(device=DEV).manual_seed(1)) if masked else None
+    got = compressed_attention(q, kc, vc, ck, cv, attention_mask=m, causal=not masked)
+    q_rot, q_proj = kc.prepare_queries(q)
+    packed = attention_from_prepared(q_rot, q_proj, kc, vc, ck, cv, attention_mask=m, causal=not masked)
+    direct = _direct(q, kc, vc, ck, cv, mask=m, causal=not masked)
+    assert torch.equal(got, direct if expanded else packed)
+    assert not torch.equal(packed, direct) and _err(direct, packed.double()) < REL
+
+
 def test_prefill_rows_without_a_real_key():
     """A row whose mask is finfo.min everywhere attends all keys equally, as softmax does."""
     kc, vc, q, ck, cv = _make(128, 3, 3, 8, 2, 70, 100)

@@ -18,6 +18,7 @@
 #include <c10/core/DeviceGuard.h>
 #include <torch/library.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <tuple>
 
@@ -579,20 +580,39 @@ bool prefill_route(int64_t B, int64_t Hq, int64_t hkv, int64_t Sq, int64_t sk, i
   if (causal && sk < Sq) return false;
   const int64_t G = Hq / hkv;
   if (G > 128 || D < 8 || D > 256 || D % 8 != 0) return false;
-  // Few columns (query rows x group) per kv head over many keys stay on the kernels that read the
-  // packed planes once, split over keys: expanding a key costs about as much as scoring it for 64
-  // columns there (32/8 heads, head_dim 128, 16 rows x 4k keys: 42 us packed, 69 us expanded; 24
-  // rows, past one block of those kernels: 205 us packed, 70 us expanded).  Those kernels split from
-  // 512 keys on and up to 128 columns (64 under a mask or above head_dim 64 without the prefill
-  // kernel); below 512 keys expanded is level at 64 columns and ahead from there.
+  // Columns: query rows x group, per kv head.  From 512 keys on the packed kernels split the keys of up
+  // to 128 columns (64 under a mask, or above head_dim 64 without the prefill kernel) and read each once:
+  // expanding a key costs about as much as scoring it for 64 columns there (32/8 heads, head_dim 128, 16
+  // rows x 4k keys: 42 us packed, 69 expanded; 24 rows, past one block of those kernels: 205 and 70).
+  const int64_t cols = G * Sq;
   const bool own = (D == 64 || D == 128) && bits == val_bits;  // the prefill kernel's shapes
-  const bool two_blocks = own ? !masked : D <= 64;
-  // Under a mask the prefill kernel's 64-column blocks are level while they leave the chip's 512
-  // block slots partly idle (32/32 heads, 500 rows: 82 us packed, 86 us expanded; 4 x 12 heads, 1000
-  // rows: 109 and 94 us)
-  if (own && masked && sk <= 1024 && B * hkv * ((G * Sq + 63) / 64) <= 512) return false;
-  const int64_t split_cols = two_blocks ? 128 : 64;
-  return sk >= 512 ? G * Sq > split_cols : G * Sq >= 64;
+  const int64_t split_cols = (own ? !masked : D <= 64) ? 128 : 64;
+  if (cols < 64 || (sk >= 512 && cols <= split_cols)) return false;
+  if (!own) return true;  // the tiled kernel: expanded is level at 64 columns and ahead from there
+  const int64_t groups = B * hkv;
+  // the tiled kernel split over keys, for want of a masked prefill kernel of more than 64 columns
+  // (head_dim 64, 100 rows, 192 (batch, kv head)s x 2000 keys: 310 us packed, 146 expanded)
+  if (masked && D == 64 && sk >= 512 && cols <= 128 && groups <= 512) return true;
+  // The prefill kernel: microseconds of both, from the query blocks that share the chip's 512 places
+  // (128 columns, 64 under a mask) and their 32-key tiles, and from the expanded elements and the columns
+  // that meet them; expanded keys past 40 million elements (240 MB) outgrow the last-level cache.  Fitted
+  // to 2,600 shapes (1 to 48 sequences, 2 to 12 kv heads, 64 to 5000 columns, up to 16k keys), 12% rms: of
+  // 3,529 shapes timed on both paths 101 are sent to a path slower by more than 4%, the worst by 1.33.  Few long blocks leave the packed grid idle (32/8 heads, head_dim 128, 33 rows
+  // x 20k keys: 850 us packed, 110 expanded); where many sequences fill it, expanding every key for a few
+  // hundred columns costs more than it saves (48 sequences of 12 heads, 200 rows x 2000 keys: 405 and
+  // 706 us; 64 rows x 500 keys: 120 and 176).
+  struct Cost {
+    double block, tile, least, call, col;  // packed: us per block and tile, least share of the chip; expanded
+  };
+  const Cost c = masked ? (D == 64 ? Cost{12, 1.4, 0.83, 28, 12.4e-3} : Cost{26, 2.75, 0.55, 37, 12.4e-3})
+                        : (D == 64 ? Cost{22, 1.8, 0.47, 24, 7.3e-3} : Cost{50, 2.95, 0.45, 34, 7.3e-3});
+  const double keys = static_cast<double>(sk) - (causal ? 0.5 * static_cast<double>(Sq) : 0.0);
+  const double blocks = static_cast<double>(groups * ((cols + split_cols - 1) / split_cols));
+  const double packed = 15 + (c.block + c.tile * keys / 32) * std::max(c.least, blocks / 512);
+  const double elements = 1e-6 * static_cast<double>(groups * D) * static_cast<double>(sk);
+  const double expanded = c.call + 3.1 * elements + 2 * std::max(0.0, elements - 40) +
+                          c.col * static_cast<double>(cols) * elements * keys / static_cast<double>(sk);
+  return expanded < packed;
 }
 
 // Attention of raw queries: the checks, and the [B, Sq, Hq, D] output
