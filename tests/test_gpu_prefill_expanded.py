@@ -276,6 +276,21 @@ def test_norms_that_are_not_finite(d, hq, hkv, sq, sk, masked):
         assert _err(got[~bad], want[~bad].double()) < REL
 
 
+@pytest.mark.parametrize("B,d,sq,sk,expanded", [(1, 192, 130, 600, True), (64, 192, 130, 700, False),
+                                                (64, 192, 170, 700, True), (64, 128, 130, 700, True),
+                                                (1, 192, 128, 700, False)])
+def test_scores_route(B, d, sq, sk, expanded):
+    """As test_prefill_route, for materialised scores (12 heads)."""
+    kc, _, q, ck, _ = _make(d, 3, 3, 12, 12, sq, sk, B=B)
+    t = _tables(kc, q.device, True)
+    packed = scores_from_prepared(*kc.prepare_queries(q), ck["packed_key_indices"], ck["packed_qjl_signs"],
+                                  ck["residual_norm"], ck["vec_norms"], t.cent16, 3, math.sqrt(math.pi / 2) / d, 12,
+                                  sk, sk)
+    got = kc.asymmetric_attention_scores(q, ck)
+    assert torch.equal(got, packed) != expanded
+    assert ((got - packed).norm() / packed.norm()).item() < 4e-5
+
+
 @pytest.mark.parametrize("d,sq,sk", [(128, 64, 96), (64, 140, 75), (80, 140, 64), (256, 140, 96)])
 def test_expanded_scores_over_all_norms(d, sq, sk):
     """Every key's scores at f32 grade whatever its neighbours' norms (f16's whole range in a tile), and
@@ -317,6 +332,8 @@ def test_expanded_scores_over_all_norms(d, sq, sk):
     (48, 64, 12, 12, 96, 1500, True, False),
     (1, 128, 32, 8, 40, 900, True, True),
     (1, 80, 32, 32, 64, 300, False, True),      # no prefill kernel
+    (48, 192, 12, 12, 64, 500, True, False),    # many wide keys for 64 columns
+    (48, 192, 12, 12, 100, 500, True, True),
 ])
 def test_prefill_route(B, d, hq, hkv, sq, sk, masked, expanded):
     """Which kernels a call takes, on both sides of each line of the rule: bit for bit those of the path

@@ -588,8 +588,13 @@ bool prefill_route(int64_t B, int64_t Hq, int64_t hkv, int64_t Sq, int64_t sk, i
   const bool own = (D == 64 || D == 128) && bits == val_bits;  // the prefill kernel's shapes
   const int64_t split_cols = (own ? !masked : D <= 64) ? 128 : 64;
   if (cols < 64 || (sk >= 512 && cols <= split_cols)) return false;
-  if (!own) return true;  // the tiled kernel: expanded is level at 64 columns and ahead from there
   const int64_t groups = B * hkv;
+  const double elements = 1e-6 * static_cast<double>(groups * D) * static_cast<double>(sk);
+  // The tiled kernel: expanded is level at 64 columns and ahead from there, but for the expansion of many
+  // wide keys (under 512 of them per sequence: above, 64 columns are split) for one block of columns
+  // (head_dim 256, 384 (batch, kv head)s x 500 keys, 64 columns under a mask: 360 us packed, 446 expanded;
+  // x 300 keys 308 and 308; 100 columns x 300 keys 565 and 353)
+  if (!own) return !(D > 160 && cols < 100 && elements > 45);
   // the tiled kernel split over keys, for want of a masked prefill kernel of more than 64 columns
   // (head_dim 64, 100 rows, 192 (batch, kv head)s x 2000 keys: 310 us packed, 146 expanded)
   if (masked && D == 64 && sk >= 512 && cols <= 128 && groups <= 512) return true;
@@ -609,7 +614,6 @@ bool prefill_route(int64_t B, int64_t Hq, int64_t hkv, int64_t Sq, int64_t sk, i
   const double keys = static_cast<double>(sk) - (causal ? 0.5 * static_cast<double>(Sq) : 0.0);
   const double blocks = static_cast<double>(groups * ((cols + split_cols - 1) / split_cols));
   const double packed = 15 + (c.block + c.tile * keys / 32) * std::max(c.least, blocks / 512);
-  const double elements = 1e-6 * static_cast<double>(groups * D) * static_cast<double>(sk);
   const double expanded = c.call + 3.1 * elements + 2 * std::max(0.0, elements - 40) +
                           c.col * static_cast<double>(cols) * elements * keys / static_cast<double>(sk);
   return expanded < packed;
@@ -681,11 +685,14 @@ Tensor attend(const Tensor& q_in, const Tensor& pi_split, const Tensor& s_eff16,
 // Materialised scores of raw queries: tq_prefill_scores past the 128 columns (query rows x group) per
 // kv head that one block of the packed-plane kernels holds (32/8 heads: 33 rows x 4096 keys 371 us
 // packed, 39 expanded; up to 128 columns those split the keys and read them once), otherwise query_prep
-// and scores.
+// and scores.  Above head_dim 128 the expansion of many keys costs more than a second visit to the packed
+// ones (head_dim 192, 512 (batch, kv head)s x 3000 keys: 132 columns 908 us packed, 1281 expanded; 160
+// 987 and 1365; 200 1334 and 1478; 64 groups: 246 and 217; head_dim 160 from 128 groups on: 225 and 257).
 bool score_route(int64_t B, int64_t Hq, int64_t hkv, int64_t Sq, int64_t sk, int64_t D, int64_t bits) {
   if (B < 1 || Hq < 1 || Sq < 1 || sk < 1 || sk >= (int64_t{1} << 24) || bits < 2 || bits > 4) return false;
   if (D < 8 || D > 256 || D % 8 != 0) return false;
-  return Hq / hkv * Sq > 128;
+  const int64_t cols = Hq / hkv * Sq;
+  return cols > 128 && !(D > 128 && cols <= 160 && 1e-6 * static_cast<double>(B * hkv * D) * static_cast<double>(sk) > 60);
 }
 
 Tensor attend_scores_meta(const Tensor& q, const Tensor& pi_split, const Tensor& s_eff16, const Tensor& codes,
