@@ -291,6 +291,33 @@ def test_scores_route(B, d, sq, sk, expanded):
     assert ((got - packed).norm() / packed.norm()).item() < 4e-5
 
 
+@pytest.mark.parametrize("d,group,masked,ok", [
+    (128, 128, False, True), (128, 136, False, False), (128, 72, True, False), (128, 64, True, True),
+    (64, 128, True, True), (64, 136, False, False), (80, 64, False, True), (80, 72, False, False),
+])
+def test_group_sizes(d, group, masked, ok):
+    """The largest GQA group does not depend on the route: what the packed kernels refuse is refused."""
+    kc, vc, q, ck, cv = _make(d, 3, 3, group, 1, 3, 70, B=1)
+    m = torch.zeros(1, 1, 3, 70, device=DEV) if masked else None
+    for split_k in (True, False):
+        if ok:
+            assert _err(compressed_attention(q, kc, vc, ck, cv, attention_mask=m, split_k=split_k),
+                        _reference(q, kc, vc, ck, cv)) < REL
+        else:
+            with pytest.raises(RuntimeError, match="group size"):
+                compressed_attention(q, kc, vc, ck, cv, attention_mask=m, split_k=split_k)
+
+
+@pytest.mark.parametrize("d,group,ok", [(128, 128, True), (128, 136, False), (160, 64, True), (160, 72, False)])
+def test_group_sizes_of_scores(d, group, ok):
+    kc, _, q, ck, _ = _make(d, 3, 3, group, 1, 3, 70, B=1)
+    if ok:
+        assert kc.asymmetric_attention_scores(q, ck).shape == (1, group, 3, 70)
+    else:
+        with pytest.raises(RuntimeError, match="group size"):
+            kc.asymmetric_attention_scores(q, ck)
+
+
 @pytest.mark.parametrize("d,sq,sk", [(128, 64, 96), (64, 140, 75), (80, 140, 64), (256, 140, 96)])
 def test_expanded_scores_over_all_norms(d, sq, sk):
     """Every key's scores at f32 grade whatever its neighbours' norms (f16's whole range in a tile), and

@@ -579,7 +579,7 @@ bool prefill_route(int64_t B, int64_t Hq, int64_t hkv, int64_t Sq, int64_t sk, i
   if (B < 1 || Hq < 1 || Sq < 1 || sk < 1 || bits < 2 || bits > 4 || val_bits < 1 || val_bits > 4) return false;
   if (causal && sk < Sq) return false;
   const int64_t G = Hq / hkv;
-  if (G > 128 || D < 8 || D > 256 || D % 8 != 0) return false;
+  if (D < 8 || D > 256 || D % 8 != 0) return false;
   // Columns: query rows x group, per kv head.  From 512 keys on the packed kernels split the keys of up
   // to 128 columns (64 under a mask, or above head_dim 64 without the prefill kernel) and read each once:
   // expanding a key costs about as much as scoring it for 64 columns there (32/8 heads, head_dim 128, 16
@@ -587,6 +587,8 @@ bool prefill_route(int64_t B, int64_t Hq, int64_t hkv, int64_t Sq, int64_t sk, i
   const int64_t cols = G * Sq;
   const bool own = (D == 64 || D == 128) && bits == val_bits;  // the prefill kernel's shapes
   const int64_t split_cols = (own ? !masked : D <= 64) ? 128 : 64;
+  // GQA groups past one block of the packed kernels are refused there, and so by every route
+  if (G > (D <= 64 ? 128 : split_cols)) return false;
   if (cols < 64 || (sk >= 512 && cols <= split_cols)) return false;
   const int64_t groups = B * hkv;
   const double elements = 1e-6 * static_cast<double>(groups * D) * static_cast<double>(sk);
@@ -691,6 +693,7 @@ Tensor attend(const Tensor& q_in, const Tensor& pi_split, const Tensor& s_eff16,
 bool score_route(int64_t B, int64_t Hq, int64_t hkv, int64_t Sq, int64_t sk, int64_t D, int64_t bits) {
   if (B < 1 || Hq < 1 || Sq < 1 || sk < 1 || sk >= (int64_t{1} << 24) || bits < 2 || bits > 4) return false;
   if (D < 8 || D > 256 || D % 8 != 0) return false;
+  if (Hq / hkv > (D <= 128 ? 128 : 64)) return false;  // groups that the packed kernel refuses
   const int64_t cols = Hq / hkv * Sq;
   return cols > 128 && !(D > 128 && cols <= 160 && 1e-6 * static_cast<double>(B * hkv * D) * static_cast<double>(sk) > 60);
 }
