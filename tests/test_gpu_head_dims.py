@@ -179,10 +179,11 @@ def test_attention_any_dim(d, bits, hq, hkv, sq, sk, causal):
     kc = TurboQuantCompressorV2(d, bits, seed=42, device=DEV)
     vc = TurboQuantCompressorMSE(d, bits, seed=10042, device=DEV)
     ck, cv = kc.compress(k), vc.compress(v)
-    got = _np(compressed_attention(q, kc, vc, ck, cv, causal=causal, out_dtype=torch.float32))
     ref = _oracle_attention(kc, vc, q, ck, cv, hq, hkv, causal=causal)
-    assert got.shape == ref.shape
-    assert O.rel_err(got, ref) < REL and O.cosine(got, ref) > 0.9999
+    for split_k in (True, False):  # many columns: expanded keys, then the tiled kernel
+        got = _np(compressed_attention(q, kc, vc, ck, cv, causal=causal, out_dtype=torch.float32, split_k=split_k))
+        assert got.shape == ref.shape
+        assert O.rel_err(got, ref) < REL and O.cosine(got, ref) > 0.9999, split_k
 
 
 @pytest.mark.parametrize("d", [80, 112, 192])

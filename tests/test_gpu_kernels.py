@@ -293,12 +293,14 @@ def _oracle_attention(kc, vc, q, ck, cv, hq, hkv, mask=None, causal=False):
     (128, 3, 32, 8, 70, 70, True), (128, 3, 8, 2, 1, 300, False), (128, 2, 4, 4, 64, 64, True),
     (128, 4, 16, 2, 33, 97, True), (64, 3, 12, 12, 40, 40, False), (32, 3, 4, 2, 20, 20, True),
     (256, 3, 4, 4, 24, 50, True),
-    # head_dim-128 prefill kernel: GQA groups that leave columns of a block unused (G=3) or give
+    # head_dim-128 kernels: GQA groups that leave columns of a block unused (G=3) or give
     # 16 query rows per block (G=8), MHA non-causal with Sk > Sq, several causal blocks at bits 2 and 4
     (128, 2, 12, 4, 50, 50, True), (128, 3, 32, 4, 20, 300, True), (128, 4, 8, 8, 40, 90, False),
     (128, 2, 4, 2, 130, 130, True), (128, 4, 8, 2, 97, 160, True),
 ])
 def test_attention_matches_oracle(d, bits, hq, hkv, sq, sk, causal):
+    """By the default route (many columns per kv head: expanded keys) and with split_k=False (the packed
+    prefill and tiled kernels)."""
     _case(d=d, bits=bits, hq=hq, hkv=hkv, sq=sq, sk=sk, causal=causal)
     torch.manual_seed(sq + 7 * sk + d)
     q = torch.randn(2, hq, sq, d, device=DEV, dtype=torch.bfloat16)
@@ -307,10 +309,11 @@ def test_attention_matches_oracle(d, bits, hq, hkv, sq, sk, causal):
     kc = TurboQuantCompressorV2(d, bits, seed=42, device=DEV)
     vc = TurboQuantCompressorMSE(d, bits, seed=10042, device=DEV)
     ck, cv = kc.compress(k), vc.compress(v)
-    got = _np(compressed_attention(q, kc, vc, ck, cv, causal=causal, out_dtype=torch.float32))
     ref = _oracle_attention(kc, vc, q, ck, cv, hq, hkv, causal=causal)
-    assert got.shape == ref.shape
-    assert O.rel_err(got, ref) < REL and O.cosine(got, ref) > 0.9999
+    for split_k in (True, False):
+        got = _np(compressed_attention(q, kc, vc, ck, cv, causal=causal, out_dtype=torch.float32, split_k=split_k))
+        assert got.shape == ref.shape
+        assert O.rel_err(got, ref) < REL and O.cosine(got, ref) > 0.9999, split_k
 
 
 @pytest.mark.parametrize("d", [64, 128])
@@ -394,9 +397,10 @@ def test_attention_left_padding_mask(bits, npad):
 
 
 @pytest.mark.parametrize("bits,sq,sk,causal,masked", [
-    (3, 160, 160, True, False),   # head_dim-128 prefill kernel, causal
-    (2, 96, 224, False, False),   # prefill kernel, Sk > Sq
+    (3, 160, 160, True, False),   # expanded keys and (split_k=False) the prefill kernel, causal
+    (2, 96, 224, False, False),   # the same, Sk > Sq
     (3, 160, 160, True, True),    # the prefill kernel's additive-mask form
+    (3, 160, 1120, True, True),   # expanded keys under a mask
     (3, 1, 2048, False, False),   # split-K decode kernels (bit-plane keys), 3 bits
     (2, 1, 2048, False, False),   # split-K decode kernels, 2 bits
 ])
@@ -420,13 +424,14 @@ def test_attention_rising_scores_rescale(bits, sq, sk, causal, masked):
         mask = torch.triu(torch.full((sq, sk), torch.finfo(torch.float32).min), 1 + sk - sq) + 0.5 * torch.randn(sq, sk)
         mask = mask[None, None]
         ref = _oracle_attention(kc, vc, q, ck, cv, hq, hkv, mask=mask.numpy())
-        got = compressed_attention(q, kc, vc, ck, cv, attention_mask=mask.to(DEV), out_dtype=torch.float32)
+        kw = dict(attention_mask=mask.to(DEV))
     else:
         ref = _oracle_attention(kc, vc, q, ck, cv, hq, hkv, causal=causal)
-        got = compressed_attention(q, kc, vc, ck, cv, causal=causal, out_dtype=torch.float32)
-    got = _np(got.float())
-    assert got.shape == ref.shape
-    assert O.rel_err(got, ref) < REL and O.cosine(got, ref) > 0.9999
+        kw = dict(causal=causal)
+    for split_k in (True, False):
+        got = _np(compressed_attention(q, kc, vc, ck, cv, out_dtype=torch.float32, split_k=split_k, **kw))
+        assert got.shape == ref.shape
+        assert O.rel_err(got, ref) < REL and O.cosine(got, ref) > 0.9999, split_k
 
 
 def test_attention_full_size_slice():

@@ -131,7 +131,9 @@ def test_prefill_shapes(d, bits, vbits, hq, hkv, sq, sk, causal):
 @pytest.mark.parametrize("sk,layout", [(160, "batch"), (161, "batch"), (200, "head"), (96, "strided")])
 def test_prefill_masks(d, mdt, sk, layout):
     """Additive masks in their own type: broadcast over heads, per head, rows that start off a
-    dword (odd key counts), and a layout that is not contiguous in keys."""
+    dword (odd key counts), and a layout that is not contiguous in keys.  Through the operator, whose
+    rule keeps so few keys at head_dim 64 and 128 on the packed prefill kernel, and through the C entry,
+    which has no rule and reads the mask where it lies."""
     print("case:", d, mdt, sk, layout, flush=True)
     sq, hq, hkv, B = 100, 8, 2, 2
     kc, vc, q, ck, cv = _make(d, 3, 3, hq, hkv, sq, sk)
@@ -141,8 +143,41 @@ def test_prefill_masks(d, mdt, sk, layout):
     m[1, :, 5:9, 40:] = -math.inf
     if layout == "strided":
         m = m.transpose(-1, -2).contiguous().transpose(-1, -2)
-    got = compressed_attention(q, kc, vc, ck, cv, attention_mask=m)
-    assert _err(got, _reference(q, kc, vc, ck, cv, mask=m.expand(B, hq, sq, sk))) < REL
+    ref = _reference(q, kc, vc, ck, cv, mask=m.expand(B, hq, sq, sk))
+    assert _err(compressed_attention(q, kc, vc, ck, cv, attention_mask=m), ref) < REL
+    assert _err(_direct(q, kc, vc, ck, cv, mask=m), ref) < REL
+
+
+def _split(B, hq, hkv, sq, sk, d):
+    """Whether a masked call's keys are split over blocks: its workspace then holds partial sums."""
+    dp, tiles = (d + 31) // 32 * 32, (sk + 31) // 32
+    q_part = 2 * dp * dp + (B * hq * sq * d * 2 + 255) // 256 * 256
+    group = (_native.lib().tq_prefill_workspace_size(B, hq, hkv, sq, sk, d, 0, 1) - q_part) // (B * hkv)
+    return group > (4 * tiles + 15) // 16 * 16 + tiles * (3 * dp * 64 + 256)
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("mdt", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,hq,hkv,sq,sk,split,causal", [
+    (2, 8, 2, 40, 3000, True, False),     # keys split over blocks and merged
+    (2, 8, 2, 40, 3000, True, True),
+    (16, 16, 16, 130, 2304, False, False),  # a block of 72 tiles: the tile factors are loaded anew after 64
+    (16, 16, 16, 130, 2304, False, True),
+])
+def test_prefill_masks_of_long_calls(d, mdt, B, hq, hkv, sq, sk, split, causal):
+    """The masked kernels over many tiles, through the C entry: left padding by finfo.min, whole rows
+    and whole key ranges of a split without a real key, -inf, with and without a causal limit."""
+    print("case:", d, mdt, B, sq, sk, causal, flush=True)
+    kc, vc, q, ck, cv = _make(d, 3, 3, hq, hkv, sq, sk, B=B)
+    assert _split(B, hq, hkv, sq, sk, d) == split
+    low = torch.finfo(mdt).min
+    m = torch.randn(B, 1, sq, sk, device=DEV, generator=torch.Generator(device=DEV).manual_seed(d)).to(mdt)
+    m[0, :, :, : sk // 2] = low
+    if mdt != torch.float16:  # f16's lowest value leaves 2^-7 of a score in f32
+        m[1, :, 3] = low
+    m[1, :, 5:9, 40:] = -math.inf
+    ref = _reference(q, kc, vc, ck, cv, mask=m.expand(B, hq, sq, sk), causal=causal)
+    assert _err(_direct(q, kc, vc, ck, cv, mask=m, causal=causal), ref) < REL
 
 
 @pytest.mark.parametrize("d", [64, 80, 128])
@@ -310,6 +345,7 @@ def test_group_sizes(d, group, masked, ok):
 
 @pytest.mark.parametrize("d,group,ok", [(128, 128, True), (128, 136, False), (160, 64, True), (160, 72, False)])
 def test_group_sizes_of_scores(d, group, ok):
+    """As test_group_sizes, for materialised scores."""
     kc, _, q, ck, _ = _make(d, 3, 3, group, 1, 3, 70, B=1)
     if ok:
         assert kc.asymmetric_attention_scores(q, ck).shape == (1, group, 3, 70)
@@ -376,14 +412,16 @@ def test_prefill_route(B, d, hq, hkv, sq, sk, masked, expanded):
     assert not torch.equal(packed, direct) and _err(direct, packed.double()) < REL
 
 
-def test_prefill_rows_without_a_real_key():
+@pytest.mark.parametrize("d", [64, 128])
+def test_prefill_rows_without_a_real_key(d):
     """A row whose mask is finfo.min everywhere attends all keys equally, as softmax does."""
-    kc, vc, q, ck, cv = _make(128, 3, 3, 8, 2, 70, 100)
+    kc, vc, q, ck, cv = _make(d, 3, 3, 8, 2, 70, 100)
     m = torch.zeros(2, 1, 70, 100, device=DEV)
     m[0, :, 3] = torch.finfo(torch.float32).min
     m[1, :, :, 50:] = torch.finfo(torch.float32).min
-    got = compressed_attention(q, kc, vc, ck, cv, attention_mask=m)
-    assert _err(got, _reference(q, kc, vc, ck, cv, mask=m.expand(2, 8, 70, 100))) < REL
+    ref = _reference(q, kc, vc, ck, cv, mask=m.expand(2, 8, 70, 100))
+    for got in (compressed_attention(q, kc, vc, ck, cv, attention_mask=m), _direct(q, kc, vc, ck, cv, mask=m)):
+        assert _err(got, ref) < REL
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
@@ -534,3 +572,21 @@ def test_expanded_scores(d, bits, hq, hkv, sq, sk, dtype):
     torch.cuda.synchronize()
     assert st == 0 and (buf[:guard] == 7).all() and (buf[-guard:] == 7).all()
     assert torch.equal(buf[guard:-guard].view(ref.shape), got)
+
+
+def test_expanded_scores_past_64_tiles():
+    """Blocks of more than 64 key tiles load the tile factors anew: 96 (batch, kv head)s of 2048 rows are
+    1536 blocks of 128 rows, and about eight blocks per compute unit leave 67 of the 90 tiles to one."""
+    B, hkv, sq, sk, d = 8, 12, 2048, 2880, 32
+    kc, _, q, ck, _ = _make(d, 3, 3, hkv, hkv, sq, sk, dtype=torch.bfloat16, B=B,
+                            scale=lambda n: torch.linspace(0.5, 40, n, device=DEV)[:, None])
+    got = kc.asymmetric_attention_scores(q, ck)
+    t = _tables(kc, q.device, True)
+    r, p = kc.prepare_queries(q[:, :, :64])
+    want = scores_from_prepared(r, p, ck["packed_key_indices"], ck["packed_qjl_signs"], ck["residual_norm"],
+                                ck["vec_norms"], t.cent16, 3, math.sqrt(math.pi / 2) / d, hkv, sk, sk)
+    assert ((got[:, :, :64] - want).norm() / want.norm()).item() < 2e-5
+    r, p = kc.prepare_queries(q[:, :, -33:])
+    want = scores_from_prepared(r, p, ck["packed_key_indices"], ck["packed_qjl_signs"], ck["residual_norm"],
+                                ck["vec_norms"], t.cent16, 3, math.sqrt(math.pi / 2) / d, hkv, sk, sk)
+    assert ((got[:, :, -33:] - want).norm() / want.norm()).item() < 2e-5
