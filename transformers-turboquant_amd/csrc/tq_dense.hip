@@ -22,13 +22,14 @@
 // one for the lo product, and the kernels take its scores over a separate, slower branch.
 //
 // Bound and measurements (bits 3, 32 / 8 heads, head_dim 128, against tq_query_prep and the
-// term-by-term prefill kernel, one MI355X): 8192 causal rows 1160 -> 815 us for the whole layer,
-// the attention kernel 1110 -> 730 us, 1.15 PFLOP/s on the matrix cores where a large library
-// product reaches 1.3 (both hold the clock below 2 GHz); 512 rows over 16k cached keys 731 -> 245
+// term-by-term prefill kernel, one MI355X): 8192 causal rows 1154-1252 -> 830-874 us for the whole layer,
+// the attention kernel 760-865 of them, 0.97-1.1 PFLOP/s on the matrix cores where a large library
+// product reaches 1.23 (both hold the clock below 2 GHz); 512 rows over 16k cached keys 734 -> 241-254
 // us (blocks split the keys, the term-by-term kernel ran 128 blocks); head_dim 80, 1531 rows, 32
-// heads: 247 -> 95 us without the compressions.  A tile takes a compute unit 0.90 us with two
+// heads: 247 -> 80 us without the compressions.  A tile takes a compute unit 0.90 us with two
 // waves per SIMD (its matrix work alone 0.64 at 2.4 GHz); the rest is the chain scores -> softmax ->
-// P.V and the barrier.  Expansion is bound by its 6 bytes written per element (8 us per 16 MB).
+// P.V and the barrier.  The expansion writes 6 bytes per element at about 2.7 TB/s (131k keys x 128: 37
+// us; a copy of as much runs at 5.1): see dense_expand_kernel.
 #include "tq_common.h"
 #include "tq_stream.h"
 
@@ -89,6 +90,9 @@ constexpr int rot_blocks() { return DP <= 192 ? DP / 32 : 4; }
 // split too, 3 passes.  Blocks past a.blocks write S_eff^T as the expansion's A fragments (32-dim
 // block w, k-step s: row m is dim 32 w + perm32(m), k-slot e is S_eff row 16 s + 8 h + e), so that
 // it reads them 16 bytes per lane instead of as single halves of S_eff's columns.
+// A few thousand rows leave the chip half idle (256 rows a block: 128 blocks for 32k rows), every block
+// staging its weights first: 10 us for 8 MB of rows.  f32 rows keep both parts of a row and spill from
+// head_dim 128 on (18 VGPRs there, 44 at 192, 104 at 224, 217 at 256; bf16 at 256: 10).
 template <int DP, int DT>
 __global__ void __launch_bounds__(512) dense_rotate_kernel(RotArgs a) {
   constexpr int KS = DP / 16, NOB = rot_blocks<DP>(), NF = NOB * KS;
@@ -300,7 +304,10 @@ __global__ void __launch_bounds__(2 * DP) dense_expand_kernel(ExpandArgs a) {
 
   const int kc = d * a.kb / 8, sc = d / 8, vc = d * a.vb / 8;
   const uint32_t km = (1u << a.kb) - 1u, vm = (1u << a.vb) - 1u;
-  // a tile's packed bytes of this lane's key, fetched one tile ahead
+  // A tile's packed bytes of this lane's key, requested one tile ahead.  codes8 picks words by the
+  // lane's half, so the compiler keeps the record in scratch (48 to 76 bytes a lane) and the wait before
+  // each read back covers the request as well: the fetch is not hidden, and this chain, not the 6 bytes
+  // written per element, bounds the kernel.
   struct Raw {
     uint32_t sw[NW];
     Field32 kf, vf;
@@ -450,7 +457,8 @@ struct DenseArgs {
   int nsplit, cpt;
 };
 
-// 4 or 8 waves of 32 columns; up to head_dim 160 two waves per SIMD (256 VGPRs each), above one.
+// 4 or 8 waves of 32 columns; up to head_dim 128 two or three waves per SIMD (at most 256 VGPRs each),
+// above one.
 // RES: blocks that share a compute unit's LDS (4-wave blocks; a lone one takes a deeper ring: the
 // copies' latency is longer than one wave per SIMD takes for a tile).
 template <int DP, int NW, bool MASK, int RES>
@@ -612,7 +620,8 @@ __device__ __forceinline__ void dense_finish(const DenseArgs& a, float16v (&o)[D
 // tiles; S^T = K^ Q_rot^T (keys are MFMA rows), online softmax down the rows, O^T += V^T P^T with
 // P = f16(2^(s - m)) straight from S^T's registers.  The scores of tile t + 1 are issued with the
 // softmax of tile t, so that a wave's matrix and vector work overlap.  Records are copied into an
-// LDS ring with direct-to-LDS loads, NS - 2 tiles ahead of the scores; one block barrier per tile.
+// LDS ring with direct-to-LDS loads, LEAD tiles ahead; one block barrier per tile, or per two tiles
+// (PAIR) while no tile needs masking.
 template <int DP, int NW, bool MASK, bool PLO, int RES>
 __global__ void __launch_bounds__(64 * NW)
 __attribute__((amdgpu_waves_per_eu(DenseCfg<DP, NW, MASK, RES>::WPE)))
@@ -978,8 +987,8 @@ dense_attn_kernel(DenseArgs a) {
       // two tiles per barrier while the block's tiles need no masking (tfb: the same for its waves):
       // tiles t + 1 and t + 2 have landed, every wave is done with t - 1, so the slots of t - 2 and t - 1
       // take t + 4 and t + 5
+      // (t - tb is even here: a new 64 tiles of factors can begin at t + 2 only)
       for (; t + 2 < tfb; t += 2) {
-        if (((t + 1 - tb) & 63) == 0) factors(t + 1);
         wait_vm<(LEAD - 3) * CPW>();
         block_sync();
         issue();
@@ -1277,18 +1286,18 @@ static int device_cus() {
   return cache[dev];
 }
 
-// Block size and key splits for the smallest estimated time.  Unit: the time a compute unit takes for
-// one tile of 256 columns (two waves per SIMD; a lone 4-wave block takes kLone of it, two of them
-// kNarrow, kUnfilled where they leave some units to one).  A block adds
-// kBlock (query fragments, first copies, output rotation), a split its partial sums through memory
-// and the merge launch.
-// Blocks that fit a compute unit together (LDS, and 256 VGPRs a wave up to head_dim 160)
+// Blocks that fit a compute unit together (LDS, and 256 VGPRs a wave up to head_dim 128)
 constexpr int dense_resident(int DP, int NW, bool masked) {
   if (NW == 8) return 1;
   return masked ? (DP <= 64 ? 2 : 1) : (DP <= 64 ? 3 : DP <= 128 ? 2 : 1);
 }
 // Head dims with an 8-wave form
 constexpr bool dense_wide(int DP) { return DP == 96 || DP == 128; }
+// Block size and key splits for the smallest estimated time.  Unit: the time a compute unit takes for
+// one tile of 256 columns (two waves per SIMD; a lone 4-wave block takes kLone of it, two of them
+// kNarrow, kUnfilled where they leave some units to one).  A block adds
+// kBlock (query fragments, first copies, output rotation), a split its partial sums through memory
+// and the merge launch.
 constexpr double kLone = 0.7, kBlock = 4.0, kMergeLaunch = 4.0, kPart = 0.04, kNarrow = 1.02, kUnfilled = 0.95;
 
 static DensePlan dense_plan(int64_t groups, int G, int Sq, int Sk, int d, bool causal, bool masked, int cus) {
@@ -1384,14 +1393,14 @@ static void launch_rotate(const void* q, int dtype, int B, int Hq, int Sq, int d
                           uint16_t* seff_frag, int cus, hipStream_t s) {
   const int DP = pad_dim(d);
   RotArgs r{};
-    r.q = q; r.n = static_cast<int64_t>(B) * Hq * Sq; r.sqb = sqb; r.sqh = sqh; r.sqs = sqs;
-    r.Hq = Hq; r.Sq = Sq; r.d = d; r.pi = key_pi_split; r.seff = key_s_eff_f16;
-    r.q_rot = q_rot; r.seff_frag = seff_frag;
-    const int64_t es = dtype == TQ_F32 ? 4 : 2;
-    r.vec = reinterpret_cast<uintptr_t>(q) % 16 == 0 && (sqb * es) % 16 == 0 && (sqh * es) % 16 == 0 &&
-            (sqs * es) % 16 == 0;
-    r.blocks = static_cast<int>(std::min<int64_t>((r.n + 255) / 256, 2LL * cus));
-    const unsigned gx = r.blocks + 4;
+  r.q = q; r.n = static_cast<int64_t>(B) * Hq * Sq; r.sqb = sqb; r.sqh = sqh; r.sqs = sqs;
+  r.Hq = Hq; r.Sq = Sq; r.d = d; r.pi = key_pi_split; r.seff = key_s_eff_f16;
+  r.q_rot = q_rot; r.seff_frag = seff_frag;
+  const int64_t es = dtype == TQ_F32 ? 4 : 2;
+  r.vec = reinterpret_cast<uintptr_t>(q) % 16 == 0 && (sqb * es) % 16 == 0 && (sqh * es) % 16 == 0 &&
+          (sqs * es) % 16 == 0;
+  r.blocks = static_cast<int>(std::min<int64_t>((r.n + 255) / 256, 2LL * cus));
+  const unsigned gx = r.blocks + 4;
 #define TQ_ROT_CASE(DD)                                                                     \
   case DD: {                                                                                \
     const dim3 g(gx, (DD / 32 + rot_blocks<DD>() - 1) / rot_blocks<DD>());                  \
@@ -1399,16 +1408,16 @@ static void launch_rotate(const void* q, int dtype, int B, int Hq, int Sq, int d
     else if (dtype == TQ_F16) dense_rotate_kernel<DD, TQ_F16><<<g, 512, 0, s>>>(r);         \
     else dense_rotate_kernel<DD, TQ_BF16><<<g, 512, 0, s>>>(r);                             \
   } break;
-    switch (DP) {
-      TQ_ROT_CASE(32)
-      TQ_ROT_CASE(64)
-      TQ_ROT_CASE(96)
-      TQ_ROT_CASE(128)
-      TQ_ROT_CASE(160)
-      TQ_ROT_CASE(192)
-      TQ_ROT_CASE(224)
-      TQ_ROT_CASE(256)
-    }
+  switch (DP) {
+    TQ_ROT_CASE(32)
+    TQ_ROT_CASE(64)
+    TQ_ROT_CASE(96)
+    TQ_ROT_CASE(128)
+    TQ_ROT_CASE(160)
+    TQ_ROT_CASE(192)
+    TQ_ROT_CASE(224)
+    TQ_ROT_CASE(256)
+  }
 #undef TQ_ROT_CASE
 }
 
