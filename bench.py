@@ -642,12 +642,13 @@ def decode_step_leg(kc, vc, steps: int = 200, hq: int = HQ, hkv: int = HKV, d: i
 
 def head_dim64_leg(steps: int, warmup: int) -> dict:
     """The head_dim-64 path (GPT-2's attention, BASELINE.json configs[0]'s shape: 12 heads, bits 3)
-    through the prefill kernel at head_dim 64: one layer's compress K / V + query prep + fused attention per step,
+    through compressed_attention: one layer's compress K / V + fused attention of the raw queries per step,
     at configs[0]'s 512 tokens and at 8192 tokens (causal), HIP events around the attention call
     and around the whole step; and one decode step's attention (one query row over 4k / 32k
     cached keys) through the split-K decode kernel at head_dim 64."""
     import torch
 
+    from turboquant_pytorch import compressed_attention
     from turboquant_pytorch.compressors import TurboQuantCompressorMSE, TurboQuantCompressorV2
     from turboquant_pytorch.fused import attention_from_prepared
 
@@ -665,10 +666,9 @@ def head_dim64_leg(steps: int, warmup: int) -> dict:
             if record:
                 e[0].record()
             ck, cv = kc.compress(k), vc.compress(v)
-            q_rot, q_proj = kc.prepare_queries(q)
             if record:
                 e[1].record()
-            attention_from_prepared(q_rot, q_proj, kc, vc, ck, cv, causal=True, out_dtype=torch.bfloat16)
+            compressed_attention(q, kc, vc, ck, cv, causal=True, out_dtype=torch.bfloat16)
             if record:
                 e[2].record()
                 marks.append(e)
@@ -710,8 +710,8 @@ def head_dim64_leg(steps: int, warmup: int) -> dict:
     out["decode_step"] = decode_step_leg(kc, vc, steps=max(steps, 50), hq=h, hkv=h, d=d,
                                          shapes=((1, 4096), (1, 32768)), label="head_dim64_decode_step")
     return {"workload": f"GPT-2 attention shape: B1 x {h} heads x d{d}, bits {BITS}, causal; "
-                        "tq::prefill_kernel<64, 3, false> (q_proj as f16 hi + lo); decode steps (one query "
-                        "row over 4k / 32k cached keys) through tq::decode_attn_i8_kernel<2, 3, false, 1, 64> "
+                        "query rotation, key expansion, tq::dense_attn_kernel<64, 4, false, false, 3>; decode steps "
+                        "(one query row over 4k / 32k cached keys) through tq::decode_attn_i8_kernel<2, 3, false, 1, 64> "
                         "+ merge",
             **out}
 
@@ -784,28 +784,25 @@ def model_leg(steps: int = 3, S_model: int = 8192, bits: int = BITS) -> dict:
 
 
 def prefill_leg(kc, vc, q, k, v, steps: int, warmup: int) -> dict:
-    """Config-2 step: compress K and V, prepare queries, causal fused attention over
-    all S query rows."""
+    """Config-2 step: compress K and V, causal fused attention of all S raw query rows (query
+    rotation, key expansion and attention kernels)."""
     import torch
 
-    from turboquant_pytorch.fused import attention_from_prepared
+    from turboquant_pytorch import compressed_attention
 
     marks = []
 
     def step(record: bool):
-        e = _events(4) if record else None
+        e = _events(3) if record else None
         if record:
             e[0].record()
         ck = kc.compress(k)
         cv = vc.compress(v)
         if record:
             e[1].record()
-        q_rot, q_proj = kc.prepare_queries(q)
+        out = compressed_attention(q, kc, vc, ck, cv, causal=True, out_dtype=torch.bfloat16)
         if record:
             e[2].record()
-        out = attention_from_prepared(q_rot, q_proj, kc, vc, ck, cv, causal=True, out_dtype=torch.bfloat16)
-        if record:
-            e[3].record()
             marks.append(e)
         return out
 
@@ -821,27 +818,27 @@ def prefill_leg(kc, vc, q, k, v, steps: int, warmup: int) -> dict:
     elapsed = time.perf_counter() - t0
     RANGES.pop()
     compress_ms = sum(m[0].elapsed_time(m[1]) for m in marks) / len(marks)
-    prep_ms = sum(m[1].elapsed_time(m[2]) for m in marks) / len(marks)
-    attn_ms = sum(m[2].elapsed_time(m[3]) for m in marks) / len(marks)
+    attn_ms = sum(m[1].elapsed_time(m[2]) for m in marks) / len(marks)
     ms_per_step = elapsed / steps * 1e3
     key_heads = B * HQ * S * (S + 1) // 2
-    attn_flops = key_heads * (2 * D + 2 * D + 2 * D)  # term 1, QJL term, P.V
+    attn_flops = key_heads * (2 * D + 2 * D + 2 * D)  # expanded keys' hi and lo parts, P.V
     compress_bytes = B * HKV * S * (2 * D * 2 + key_rec_bytes(BITS, D) + val_rec_bytes(BITS, D))
     tflops = attn_flops / (attn_ms * 1e-3) / 1e12
     return {
-        "workload": f"configs[1]: causal prefill B{B} Hq{HQ} Hkv{HKV} d{D} S{S} bits{BITS}: compress K/V + query prep + "
-                    "fused scores/softmax/P.V",
+        "workload": f"configs[1]: causal prefill B{B} Hq{HQ} Hkv{HKV} d{D} S{S} bits{BITS}: compress K/V + fused "
+                    "attention of the raw queries",
         "ms_per_step": ms_per_step,
         "key_heads_per_s": key_heads / (ms_per_step * 1e-3),
         "compress_tokens_per_s": B * S / (compress_ms * 1e-3),
         "compress_ms": compress_ms,
         "compress_hbm_gbs": compress_bytes / (compress_ms * 1e-3) / 1e9,
-        "query_prep_ms": prep_ms,
         "attention_ms": attn_ms,
         "roofline": {
-            "kernel": "tq::prefill_kernel<128, 3, false> (fused scores + softmax + P.V; q_proj as f16 hi + lo)",
+            "kernel": "tq::dense_attn_kernel<128, 8, false, false, 1> (scores + softmax + P.V; timed with the query "
+                      "rotation and the key expansion before it)",
             "bound": "mfma", "achieved": tflops, "peak": MFMA_F16_PEAK_TFLOPS, "unit": "TFLOP/s",
-            "frac": tflops / MFMA_F16_PEAK_TFLOPS, "traffic": measured_traffic("tq::prefill_kernel<128, 3, false>"),
+            "frac": tflops / MFMA_F16_PEAK_TFLOPS,
+            "traffic": measured_traffic("tq::dense_attn_kernel<128, 8, false, false, 1>"),
         },
     }
 
