@@ -229,8 +229,9 @@ int tq_attention_fwd_kv(const uint16_t* q_rot, const float* q_proj,
  *   k^ = vn Ck[codes] + coeff rn S_eff^T (2*sign - 1),   score = <q_rot, k^>,
  * (f32 grade: f16 hi + lo parts) instead of projecting every query; key_s_eff_f16 is the same
  * f16[d, d] table tq_query_prep takes.  Other operands as in tq_attention_fwd_kv; the mask is
- * read in its own type (mask_dtype); out is contiguous [B, Sq, Hq, d].  `workspace` (16-byte
- * aligned) holds the rotated queries and the expanded keys and values:
+ * read in its own type (mask_dtype), fastest where its rows are whole dwords and contiguous in
+ * keys; out is contiguous [B, Sq, Hq, d].  out, key_pi_split, val_pit_split and `workspace` are
+ * 16-byte aligned; the workspace holds the rotated queries and the expanded keys and values:
  * tq_prefill_workspace_size bytes run every (batch, kv head) at once up to 1 GiB of expanded
  * planes and the rest in further rounds over the same memory.
  * Replaces the family forward tail families/qwen2.py:105-117, as tq_attention_fwd. */
