@@ -1,6 +1,6 @@
 """Benchmark of the TurboQuant compressed-attention hot path on one MI355X.
 
-Headline (`value`, HBM roofline): the north-star target, compressed-key scoring
+Headline (`value`, HBM roofline): compressed-key scoring
 of Llama-3-8B-shaped attention (32 query heads, 8 KV heads, head_dim 128,
 bits 3) at 32k context, decode-shaped (keys streamed once per query step: the
 regime the metric's "% of HBM peak" refers to).  A step is one
@@ -10,13 +10,13 @@ the reference's scoring API).  Steps rotate over DEC_ROT distinct caches so the
 working set (>1 GB) is far beyond the 256 MB MALL.  The same shape is also timed
 through the fused decode attention (softmax . V).
 
-Secondary legs in the same line: BASELINE.json configs[1] (the same layer shape
+Secondary legs in the same line: a causal prompt (the same layer shape
 at 8192 tokens, bf16 Q/K/V ~ N(0,1) with 4 outlier channels x20 on K): compress
 tokens/s and the causal prefill (scores + online softmax + P.V for every query
 row, MFMA roofline); one layer's eager decode step through the product path
 (torch.ops.tq) at B = 1 with 4096 cached tokens, host and device time; the HBM
-stream ceilings; compression at the north-star scale (1M key + 1M value rows);
-the head_dim-64 (GPT-2) tiled path; and configs[2]'s 36-layer model forward
+stream ceilings; compression of 1M key + 1M value rows; the head_dim-64 (GPT-2)
+path; and the forward of a 36-layer Qwen2.5-3B-shaped model
 with its per-layer attention time.  CPU baselines: the build's torch CPU branch
 of the reference's PyTorch path on bounded samples.  Prints one JSON line.  With --gpus N > 1 it exits: this build
 runs on one GPU.
@@ -543,7 +543,7 @@ def hbm_ceiling_leg(steps: int, warmup: int) -> dict:
 
 
 def compress_leg(kc, vc, steps: int, warmup: int) -> dict:
-    """Compression at the north-star scale: keys and values of 4 sequences x 8 kv heads x 32768
+    """Compression of a million rows: keys and values of 4 sequences x 8 kv heads x 32768
     tokens (1,048,576 rows each, bf16, bits 3), timed separately with HIP events.  HBM: 256 B read
     + the record written per row (52 B keys, 50 B values).  MFMA: the f32-grade products run as
     f16 passes: a bf16 row is exact in f16 under a power-of-two row scale, so x Pi^T takes the
@@ -641,9 +641,9 @@ def decode_step_leg(kc, vc, steps: int = 200, hq: int = HQ, hkv: int = HKV, d: i
 
 
 def head_dim64_leg(steps: int, warmup: int) -> dict:
-    """The head_dim-64 path (GPT-2's attention, BASELINE.json configs[0]'s shape: 12 heads, bits 3)
+    """The head_dim-64 path (GPT-2's attention: 12 heads, bits 3)
     through compressed_attention: one layer's compress K / V + fused attention of the raw queries per step,
-    at configs[0]'s 512 tokens and at 8192 tokens (causal), HIP events around the attention call
+    at 512 tokens and at 8192 tokens (causal), HIP events around the attention call
     and around the whole step; and one decode step's attention (one query row over 4k / 32k
     cached keys) through the split-K decode kernel at head_dim 64."""
     import torch
@@ -717,7 +717,7 @@ def head_dim64_leg(steps: int, warmup: int) -> dict:
 
 
 def model_leg(steps: int = 3, S_model: int = 8192, bits: int = BITS) -> dict:
-    """the 36-layer Qwen2.5-3B-shaped random-init model (hidden 2048, 16 / 2
+    """The 36-layer Qwen2.5-3B-shaped random-init model (hidden 2048, 16 / 2
     heads, head_dim 128, bf16) patched by apply_turboquant (bits 3, seed 42, the reference's
     defaults), one full-sequence forward of 8192 uniform-random token ids with logits_to_keep=1.
     Whole-forward time (HIP events around each forward) and the time of every patched attention
@@ -776,7 +776,7 @@ def model_leg(steps: int = 3, S_model: int = 8192, bits: int = BITS) -> dict:
     attn_ms = sum(m[0].elapsed_time(m[1]) for m in marks) / steps
     del model
     torch.cuda.empty_cache()
-    return {"workload": (f"configs[2]: Qwen2.5-3B-shaped random-init model, 36 layers, bf16, B1 x {S_model} tokens, "
+    return {"workload": (f"Qwen2.5-3B-shaped random-init model, 36 layers, bf16, B1 x {S_model} tokens, "
                          f"bits {bits}, apply_turboquant defaults (non-causal as the reference), logits_to_keep=1"),
             "forward_ms": fwd_ms, "tokens_per_s": S_model / (fwd_ms * 1e-3),
             "attention_modules_ms": attn_ms, "attention_ms_per_layer": attn_ms / n_layers,
@@ -825,7 +825,7 @@ def prefill_leg(kc, vc, q, k, v, steps: int, warmup: int) -> dict:
     compress_bytes = B * HKV * S * (2 * D * 2 + key_rec_bytes(BITS, D) + val_rec_bytes(BITS, D))
     tflops = attn_flops / (attn_ms * 1e-3) / 1e12
     return {
-        "workload": f"configs[1]: causal prefill B{B} Hq{HQ} Hkv{HKV} d{D} S{S} bits{BITS}: compress K/V + fused "
+        "workload": f"causal prefill B{B} Hq{HQ} Hkv{HKV} d{D} S{S} bits{BITS}: compress K/V + fused "
                     "attention of the raw queries",
         "ms_per_step": ms_per_step,
         "key_heads_per_s": key_heads / (ms_per_step * 1e-3),
@@ -854,7 +854,7 @@ def main() -> None:
     ap.add_argument("--no-ceiling", action="store_true", help="skip the HBM stream-ceiling leg")
     ap.add_argument("--no-model", action="store_true", help="skip the whole-model forward leg")
     ap.add_argument("--compress-only", action="store_true",
-                    help="run only the north-star compression leg (1M key + 1M value rows) and print its record")
+                    help="run only the compression leg (1M key + 1M value rows) and print its record")
     ap.add_argument("--calibrate-copy", type=int, default=0, metavar="MIB",
                     help="run one device-to-device copy of MIB MiB first (PMC byte-counter calibration)")
     ap.add_argument("--pmc-summary", nargs="+", metavar="CSV",
@@ -901,7 +901,7 @@ def main() -> None:
         del src, dst
 
     if args.compress_only:
-        print(json.dumps({"compress_north_star": compress_leg(kc, vc, args.steps, args.warmup)}), flush=True)
+        print(json.dumps({"compress_1m_rows": compress_leg(kc, vc, args.steps, args.warmup)}), flush=True)
         return
 
     scores_leg, attn_leg = decode_legs(kc, vc, outliers, args.steps, args.warmup)
@@ -926,7 +926,7 @@ def main() -> None:
         "dtype": ("int8-mfma bit-plane keys x 24-bit fixed-point queries (four int8 digits, exact int32 sums: "
                   "f32-grade q_rot.C and q_proj), f32 scores"),
         "data": "synthetic (bf16 N(0,1) Q/K/V, 4 K channels x20 = randperm(128, seed 1)[:4]; seeds 0 and 2)",
-        "config": {"workload": (f"north-star target: Llama-3-8B attention (Hq{HQ} Hkv{HKV} d{D} bits{BITS}) at "
+        "config": {"workload": (f"Llama-3-8B attention (Hq{HQ} Hkv{HKV} d{D} bits{BITS}) at "
                                 f"{DEC_SK // 1024}k context, decode-shaped scoring: 1 query row x {DEC_B} sequences x "
                                 f"{DEC_SK} keys per step, rotating over {DEC_ROT} caches"),
                    "global_batch": DEC_B, "seq_len": DEC_SK, "parallelism": "single-gpu",
@@ -938,7 +938,7 @@ def main() -> None:
         "decode_attention": attn_leg,
         "prefill": prefill,
         "decode_step": None if args.no_prefill else decode_step_leg(kc, vc),
-        "compress_north_star": None if args.no_prefill else compress_leg(kc, vc, 5, 2),
+        "compress_1m_rows": None if args.no_prefill else compress_leg(kc, vc, 5, 2),
         "head_dim64": None if args.no_prefill else head_dim64_leg(args.steps, args.warmup),
         "model_forward": None if (args.no_prefill or args.no_model) else model_leg(),
     }

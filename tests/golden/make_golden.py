@@ -1,6 +1,6 @@
 """Write golden fixtures for the parts of the hot path that no closed form pins.
 
-Run in the build container only (the reference is not present on GPU boxes):
+Run where the reference's sources are:
 
     python tests/golden/make_golden.py /root/reference
 

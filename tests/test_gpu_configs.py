@@ -1,4 +1,4 @@
-"""GPU parity on the other benchmark configurations (BASELINE.json configs[2..4]).
+"""GPU parity on the other benchmark configurations.
 
 Each case runs the HIP path on the full workload of one attention layer (or one
 whole model) and checks oracle slices: the float64 oracle estimator on the
@@ -7,12 +7,12 @@ the softmax / P.V tail (families/qwen2.py:110-117, llama.py:107-122) and
 value decompression (compressors.py:311-317), within rel-err 1e-3 and cosine
 0.9999 per output row.
 
-  configs[2]  Qwen2.5-3B attention: 16 query / 2 kv heads, causal prefill of
+  Qwen2.5-3B attention: 16 query / 2 kv heads, causal prefill of
               2048 / 4096 / 8192 tokens, bits 2 / 3 / 4; and the 36-layer
               random-init model's bf16 forward at 2048 tokens
-  configs[3]  Llama-3.1-8B attention: 32 / 8 heads, 4 sequences x 32768 tokens,
+  Llama-3.1-8B attention: 32 / 8 heads, 4 sequences x 32768 tokens,
               bits 4: causal prefill and one decode step
-  configs[4]  DeepSeek-LLM-7B MHA: 32 / 32 heads, bits 2, Student-t(5) keys:
+  DeepSeek-LLM-7B MHA: 32 / 32 heads, bits 2, Student-t(5) keys:
               8 x 16384 (decode and causal prefill) and 1 x 131072 (decode)
 """
 
@@ -86,7 +86,7 @@ def _randn(shape, seed, dtype=torch.bfloat16):
     return torch.randn(*shape, device=DEV, generator=g).to(dtype)
 
 
-# ---------------------------------------------------------------- configs[2]: Qwen2.5-3B
+# ---------------------------------------------------------------- Qwen2.5-3B
 
 @pytest.mark.parametrize("bits", [2, 3, 4])
 @pytest.mark.parametrize("S", [2048, 4096, 8192])
@@ -174,7 +174,7 @@ def test_qwen25_3b_model_forward_bf16():
         assert cos > 0.99, (i, cos)
 
 
-# ---------------------------------------------------------------- configs[3]: Llama-3.1-8B
+# ---------------------------------------------------------------- Llama-3.1-8B
 
 def test_llama31_8b_layer_prefill_and_decode():
     _case(config=3, B=4, S=32768, bits=4)
@@ -199,7 +199,7 @@ def test_llama31_8b_layer_prefill_and_decode():
     _check_rows(outd, qd, kc, vc, ck, cv, hkv, [(b, h, [0]) for b in (0, 3) for h in range(hq)], causal=False)
 
 
-# ---------------------------------------------------------------- configs[4]: DeepSeek-7B MHA
+# ---------------------------------------------------------------- DeepSeek-7B MHA
 
 def _student_t(shape, seed):
     torch.manual_seed(seed)

@@ -1,4 +1,4 @@
-"""Whole-model forwards at the benchmark configurations' scale (BASELINE.json configs[2..4]).
+"""Whole-model forwards at the benchmark configurations' scale.
 
 The reference path is one family forward() per layer (families/qwen2.py:69-125,
 llama.py:18-122): q/k/v projections, rotary, compress K and V, asymmetric
@@ -14,9 +14,9 @@ full-sequence forward with logits_to_keep=1, and checks
     (reference attention.py:419-461, compressors.py:186-189, qwen2.py:110-117)
     on sampled rows, within rel-err 1e-3 and cosine 0.9999.
 
-  configs[2]  Qwen2.5-3B: 36 layers, hidden 2048, 16 / 2 heads, 4096 and 8192 tokens, bits 2 / 4
-  configs[3]  Llama-3.1-8B: 32 layers, hidden 4096, 32 / 8 heads, 4 x 32768 tokens, bits 4
-  configs[4]  DeepSeek-LLM-7B (model_type llama, MHA 32 / 32): 30 layers, 8 x 16384 tokens, bits 2
+  Qwen2.5-3B: 36 layers, hidden 2048, 16 / 2 heads, 4096 and 8192 tokens, bits 2 / 4
+  Llama-3.1-8B: 32 layers, hidden 4096, 32 / 8 heads, 4 x 32768 tokens, bits 4
+  DeepSeek-LLM-7B (model_type llama, MHA 32 / 32): 30 layers, 8 x 16384 tokens, bits 2
 """
 
 import gc

@@ -1,4 +1,4 @@
-"""Bit-exact packed codes at the north-star scale: Llama-3-8B keys and values of
+"""Bit-exact packed codes of a million rows: Llama-3-8B keys and values of
 4 sequences x 8 kv heads x 32768 positions (1M rows, head_dim 128), bits 2/3/4,
 plus GPT-2-shaped head_dim 64 at 98,304 rows and the query preparation of a
 full 8192-token prefill.
@@ -70,7 +70,7 @@ def _check_keys(x, kc, ck, y_dev, p_dev):
 
 
 @pytest.mark.parametrize("bits", [2, 3, 4])
-def test_key_codes_bit_exact_north_star(bits):
+def test_key_codes_bit_exact_1m_rows(bits):
     shape = (4, 8, 32768, 128)
     _case(what="keys", shape=shape, bits=bits)
     x = _keys(shape, seed=100 + bits)
@@ -84,7 +84,7 @@ def test_key_codes_bit_exact_north_star(bits):
 
 
 @pytest.mark.parametrize("bits", [2, 3, 4])
-def test_value_codes_bit_exact_north_star(bits):
+def test_value_codes_bit_exact_1m_rows(bits):
     shape = (4, 8, 32768, 128)
     _case(what="values", shape=shape, bits=bits)
     x = _keys(shape, seed=200 + bits, outliers=False)

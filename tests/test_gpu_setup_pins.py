@@ -1,4 +1,4 @@
-"""Compressor set-up pinned on the GPU box itself.
+"""Compressor set-up pinned on the machine that runs the model.
 
 Pi (a LAPACK QR), S (a seeded torch.randn) and the Lloyd-Max codebooks are
 computed on the host of whatever machine runs the model.  These checks repeat
