@@ -22,9 +22,9 @@
 // one for the lo product, and the kernels take its scores over a separate, slower branch.
 //
 // Bound and measurements (bits 3, 32 / 8 heads, head_dim 128, against tq_query_prep and the
-// term-by-term prefill kernel, one MI355X): 8192 causal rows 1154-1252 -> 830-874 us for the whole layer,
+// term-by-term prefill kernel, one MI355X): 8192 causal rows 1154-1364 -> 830-887 us for the whole layer,
 // the attention kernel 760-865 of them, 0.97-1.1 PFLOP/s on the matrix cores where a large library
-// product reaches 1.23 (both hold the clock below 2 GHz); 512 rows over 16k cached keys 734 -> 241-254
+// product reaches 1.23 (both hold the clock below 2 GHz); 512 rows over 16k cached keys 734 -> 241-258
 // us (blocks split the keys, the term-by-term kernel ran 128 blocks); head_dim 80, 1531 rows, 32
 // heads: 247 -> 80 us without the compressions.  A tile takes a compute unit 0.90 us with two
 // waves per SIMD (its matrix work alone 0.64 at 2.4 GHz); the rest is the chain scores -> softmax ->
